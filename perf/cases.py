@@ -10,7 +10,7 @@ unequal extents, both arithmetic precisions and the preconditioners the models a
 A state is a context with its fields in place; `run` starts from those fields every time, so
 it can be repeated.  `exact` restates each model in plain torch and FP64: on these uniform
 meshes with collocated quadrature the assembled operators are M (r(u) + beta L u), with M the
-lumped mass and L the line stencils of `_taps`; elasticity is assembled cell by cell.
+lumped mass and L the line stencils of `_Axis`; elasticity is assembled cell by cell.
 """
 
 from __future__ import annotations
