@@ -84,6 +84,20 @@ namespace ppf
     bool   alpha_constant = false;
     double alpha[PPF_MAX_FIELDS] {};
     double beta_src[PPF_MAX_FIELDS] {};
+    /// The operator of three coupled components (coupled_kernels.hpp): no value term, and
+    /// flux c, direction d, = sum coupling[c][d][s][e] times derivative e of input s with
+    /// constant coefficients.  Found only where the isotropic structure above is not.
+    bool   coupled = false;
+    int    coupled_out[3] {};
+    int    coupled_field[3] {}, coupled_slot[3] {};
+    double coupling[3][3][3][3] {};
+
+    /// A stencil path (split or coupled) takes the operator.
+    bool
+    stencil() const
+    {
+      return eligible || coupled;
+    }
   };
 
   template <class PDE, int dim, int degree, typename number>
@@ -320,6 +334,106 @@ namespace ppf
 
       plan.eligible = true;
       return plan;
+    }
+
+    /// Adds the coupled structure to a plan that `analyse` rejected: three gradient
+    /// inputs of the three output fields, gradient terms linear in the gradients with constant
+    /// coefficients, no value terms; checked on the same kind of random states, times and
+    /// increments.
+    void
+    analyse_coupled(SplitPlan &plan, double time, double dt, unsigned int inc) const
+    {
+      if constexpr (dim == 3)
+        {
+          int n_in = 0, n_out = 0;
+          for (const auto &in : inputs)
+            {
+              if (!(in.flags & slot_gradients))
+                return;
+              if (n_in == 3)
+                return;
+              plan.coupled_field[n_in]  = in.field;
+              plan.coupled_slot[n_in++] = in.slot;
+            }
+          for (int f = 0; f < PPF_MAX_FIELDS; ++f)
+            if (out_mask & (1u << f))
+              {
+                if (n_out == 3)
+                  return;
+                plan.coupled_out[n_out++] = f;
+              }
+          if (n_in != 3 || n_out != 3)
+            return;
+          // Operand c is the field that output c solves for.
+          for (int c = 0; c < 3; ++c)
+            if (plan.coupled_field[c] != plan.coupled_out[c])
+              return;
+
+          std::mt19937_64 rng(0x853c49e6748fea9bull ^ (uint64_t(block.id) * 2 + lhs));
+          for (int s = 0; s < 3; ++s)
+            for (int e = 0; e < 3; ++e)
+              {
+                State st = random_state(rng, 0.5, 0.4);
+                for (const auto &o : inputs)
+                  for (int d = 0; d < dim; ++d)
+                    st.g[o.field][o.slot][d] = number(0);
+                st.g[plan.coupled_field[s]][plan.coupled_slot[s]][e] = number(1);
+                const FC r = eval(st, time, dt, inc);
+                for (int c = 0; c < 3; ++c)
+                  for (int d = 0; d < 3; ++d)
+                    plan.coupling[c][d][s][e] = double(r.gradient_term[plan.coupled_out[c]][d]);
+              }
+
+          // An orthotropic material's coupling: direct derivatives of the own component,
+          // mixed ones between the components of their two axes.
+          for (int c = 0; c < 3; ++c)
+            for (int d = 0; d < 3; ++d)
+              for (int s = 0; s < 3; ++s)
+                for (int e = 0; e < 3; ++e)
+                  if (plan.coupling[c][d][s][e] != 0.0 &&
+                      !(d == e ? c == s : (c == d && s == e) || (c == e && s == d)))
+                    return;
+
+          const double tol   = std::is_same_v<number, float> ? 1e-5 : 1e-12;
+          const auto   check = [&](const State &st, double t, unsigned int i) {
+            const FC fc = eval(st, t, dt, i);
+            if (fc.geometry_reads)
+              return false;
+            for (int f = 0; f < PPF_MAX_FIELDS; ++f)
+              if (fc.value_term[f] != number(0))
+                return false;
+            for (int c = 0; c < 3; ++c)
+              for (int d = 0; d < 3; ++d)
+                {
+                  double pred = 0.0, scale = 0.0;
+                  for (int s = 0; s < 3; ++s)
+                    for (int e = 0; e < 3; ++e)
+                      {
+                        const double v =
+                          plan.coupling[c][d][s][e] *
+                          double(st.g[plan.coupled_field[s]][plan.coupled_slot[s]][e]);
+                        pred += v;
+                        scale += std::abs(v);
+                      }
+                  const double got = double(fc.gradient_term[plan.coupled_out[c]][d]);
+                  if (!(std::abs(got - pred) <= tol * (scale + std::abs(got)) + 1e-300))
+                    return false;
+                }
+            return true;
+          };
+          for (const double width : {0.4, 3.0, 50.0})
+            for (int k = 0; k < 3; ++k)
+              if (!check(random_state(rng, width == 0.4 ? 0.5 : 0.0, width), time, inc))
+                return;
+          // Coefficients that change with the time or the increment are not taken.
+          for (const double t : {time + 0.731, time + 13.7, 2.0 * time + 101.0})
+            if (!check(random_state(rng, 0.0, 3.0), t, inc))
+              return;
+          for (const unsigned int i : {inc + 1, inc + 3, 3u, 1000u})
+            if (!check(random_state(rng, 0.0, 3.0), time, i))
+              return;
+          plan.coupled = true;
+        }
     }
 
   private:

@@ -10,6 +10,7 @@
 // field/solve-block declarations (the body of a reference `main.cc`).
 #pragma once
 
+#include "coupled_kernels.hpp"
 #include "device.hpp"
 #include "grid.hpp"
 #include "operator_kernels.hpp"
@@ -648,19 +649,23 @@ namespace ppf
       HookProbe<PDE<number>, dim, degree, number> probe(pde, blocks[b], lhs);
       PlanEntry entry;
       entry.plan      = probe.analyse(timer.get_time(), timer.get_timestep(), timer.get_increment());
+      if (!entry.plan.eligible)
+        probe.analyse_coupled(entry.plan, timer.get_time(), timer.get_timestep(),
+                              timer.get_increment());
       ++graph_epoch;
       entry.time      = timer.get_time();
       entry.dt        = timer.get_timestep();
       entry.increment = timer.get_increment();
       // A plan that was rejected by the runtime comparison stays rejected.
-      if (it != plans.end() && !it->second.plan.eligible && it->second.verified)
+      if (it != plans.end() && !it->second.plan.stencil() && it->second.verified)
         {
           entry.plan.eligible = false;
+          entry.plan.coupled  = false;
           entry.plan.reason   = it->second.plan.reason;
           entry.verified      = true;
         }
       else if (it != plans.end())
-        entry.verified = it->second.verified && entry.plan.eligible;
+        entry.verified = it->second.verified && entry.plan.stencil();
       return plans[key] = entry, plans[key];
     }
 
@@ -797,7 +802,24 @@ namespace ppf
                                         "qualify: " + plan.reason);
       const auto        &pde = *pde_of<number>();
       const unsigned int nb  = grid_for(g.n_nodes, block_size);
-      auto launch = [&](bool split, const OutTable<number> &o) {
+      // Coupled components take the stencil in place of the one-launch generic kernels; a
+      // program that asked for the two-pass kernels keeps them.
+      const bool use_coupled = path == OperatorPath::Auto && generic_cell_block && !use_split &&
+                               takes_coupled(plan, g);
+      auto launch = [&](bool stencil, const OutTable<number> &o) {
+        if (stencil && use_coupled)
+          {
+            launch_coupled(g, deps, o, plan);
+            if (!coupled_noted.count({b, lhs}))
+              {
+                coupled_noted.insert({b, lhs});
+                log += "solve block " + std::to_string(blk.id) + " (" + (lhs ? "lhs" : "rhs") +
+                       "): coupled stencil\n";
+              }
+            PPF_HIP_CHECK(hipGetLastError());
+            return;
+          }
+        const bool split = stencil && use_split;
         dispatch_block_id(typename App::BlockIds {}, blk.id, [&](auto bid) {
           constexpr int id = decltype(bid)::value;
           if (split && path != OperatorPath::SplitNode &&
@@ -839,7 +861,8 @@ namespace ppf
       // plan is dropped (for good, with a line in the output log) if they disagree.  This
       // catches coefficients that branch on values or times the structure probe did not
       // visit.
-      if (use_split && path == OperatorPath::Auto && !entry.verified && lf.grid == &fine &&
+      if ((use_split || use_coupled) && path == OperatorPath::Auto && !entry.verified &&
+          lf.grid == &fine &&
           !std::any_of(std::begin(dst), std::end(dst),
                        [&](const number *d) {
                          for (const number *sp : src)
@@ -910,6 +933,7 @@ namespace ppf
                           << worst / std::max(scale, 1e-300)
                           << " (relative) on the current fields; using the generic path";
                       entry.plan.eligible = false;
+                      entry.plan.coupled  = false;
                       entry.plan.reason   = msg.str();
                       log += msg.str() + "\n";
                       if (std::getenv("PPF_VERBOSE"))
@@ -922,7 +946,142 @@ namespace ppf
               return;
             }
         }
-      launch(use_split, out);
+      launch(use_split || use_coupled, out);
+    }
+
+    /// Whether the coupled stencil kernel runs a plan on lattice g: 3-D Q2, at least five
+    /// nodes per axis (a halo position wraps or reflects once), arrays below 4 GiB (32-bit
+    /// byte offsets).
+    bool
+    takes_coupled(const SplitPlan &plan, const GridDesc &g) const
+    {
+      if constexpr (dim == 3 && degree == 2)
+        {
+          if (!plan.coupled)
+            return false;
+          for (int d = 0; d < 3; ++d)
+            if (g.nodes[d] < 5)
+              return false;
+          return g.n_nodes <= (int64_t(1) << 29);
+        }
+      else
+        return false;
+    }
+
+    /// Arguments of the coupled stencil kernels for lattice g.
+    template <typename number>
+    CoupledArgs<number>
+    coupled_args(const GridDesc &g, const SplitPlan &plan, int scaling) const
+    {
+      CoupledArgs<number> a {};
+      for (int d = 0; d < 3; ++d)
+        {
+          a.n[d]        = g.nodes[d];
+          a.periodic[d] = g.periodic[d];
+          for (int c = 0; c < 3; ++c)
+            {
+              const double m = class_mass_units<2>(c) * g.h[d];
+              a.sfac[d][c]   = number(scaling == scale_none ? m
+                                      : scaling == scale_invm ? 1.0 : std::sqrt(m));
+            }
+        }
+      for (int s = 0; s < 3; ++s)
+        for (int k = 0; k < 12; ++k)
+          for (int c = 0; c < 3; ++c)
+            {
+              const int  d = coupled_axes[k][0], e = coupled_axes[k][1];
+              const auto C = [&](int i, int j) {
+                return plan.coupling[c][i][s][j] / (g.h[i] * g.h[j]);
+              };
+              a.coef[s][k][c] = number(k >= 3 && k < 6 ? -(C(d, e) + C(e, d)) : C(d, e));
+            }
+      unsigned int all_dirichlet = ~0u;
+      for (int c = 0; c < 3; ++c)
+        {
+          a.dst_dmask[c] = dirichlet_mask(plan.coupled_out[c]);
+          all_dirichlet &= a.dst_dmask[c];
+        }
+      for (int d = 0; d < 3; ++d)
+        if (!g.periodic[d])
+          a.natural |= (3u << (2 * d)) & ~all_dirichlet;
+      return a;
+    }
+
+    /// Launches the coupled stencil kernel (the caller has asked takes_coupled).
+    template <typename number>
+    void
+    launch_coupled(const GridDesc &g, const DepTable<number> &deps, const OutTable<number> &out,
+                   const SplitPlan &plan)
+    {
+      if constexpr (dim == 3 && degree == 2)
+        {
+          CoupledArgs<number> a = coupled_args<number>(g, plan, out.scaling);
+          for (int s = 0; s < 3; ++s)
+            {
+              const int f   = plan.coupled_field[s], sl = plan.coupled_slot[s];
+              a.op[s]       = deps.ptr[f][sl];
+              a.op_dmask[s] = (deps.flags[f][sl] & slot_constrained) ? deps.dirichlet_mask[f] : 0u;
+              a.dst[s]      = out.dst[plan.coupled_out[s]];
+            }
+          a.keep_dirichlet = out.dirichlet_write == dirichlet_value ? 1 : 0;
+          a.halt           = out.halt;
+          const int64_t footprint = 6 * g.n_nodes * int64_t(sizeof(number));
+          a.nt_store = stencil_store_policy == StorePolicy::NonTemporal ||
+                       (stencil_store_policy == StorePolicy::Auto &&
+                        footprint > stencil_nt_min_bytes);
+          // Tile shape: the fewest workgroups, halo staging counted at a quarter of a
+          // thread's work; a lattice of 129 nodes takes 43 columns x 10 rows, where tiles
+          // of 64 columns would leave a third of the lanes idle.  At least 32 columns, so
+          // that half a wave reads consecutive words of shared memory.
+          double best = 0.0;
+          for (int tx = std::min(64, g.nodes[0]); tx >= std::min(32, g.nodes[0]); --tx)
+            {
+              const int strips = std::min(coupled_threads / tx, (g.nodes[1] + 1) / 2);
+              const int box    = (tx + 4) * (2 * strips + 4);
+              if (box > coupled_loads * coupled_threads)
+                continue;
+              const int64_t tiles = int64_t((g.nodes[0] + tx - 1) / tx) *
+                                    ((g.nodes[1] + 2 * strips - 1) / (2 * strips));
+              const double  cost  = double(tiles) * (coupled_threads + 0.25 * box);
+              if (a.tx == 0 || cost < best)
+                {
+                  best     = cost;
+                  a.tx     = tx;
+                  a.strips = strips;
+                }
+            }
+          a.tiles_x = (g.nodes[0] + a.tx - 1) / a.tx;
+          a.tiles_y = (g.nodes[1] + 2 * a.strips - 1) / (2 * a.strips);
+          // z chunk (even): a chunk marches four planes more than it owns, and the chip
+          // runs `slots` workgroups at a time, all of one length: whole rounds of them.
+          const int64_t tiles = int64_t(a.tiles_x) * a.tiles_y;
+          const int64_t slots = coupled_resident * device_cus();
+          int64_t       least = 0;
+          for (int zc = 2; zc < g.nodes[2] + 2; zc += 2)
+            {
+              const int64_t chunks = (g.nodes[2] + zc - 1) / zc;
+              const int64_t cost   = (zc + 4) * ((tiles * chunks + slots - 1) / slots);
+              if (a.z_chunk == 0 || cost < least)
+                {
+                  least     = cost;
+                  a.z_chunk = zc;
+                }
+            }
+          if (column_chunk > 0)
+            a.z_chunk = 2 * column_chunk;
+          a.chunks_z = (g.nodes[2] + a.z_chunk - 1) / a.z_chunk;
+          const int64_t nblocks = tiles * a.chunks_z;
+          if (nblocks >= (int64_t(1) << 31))
+            throw Error(status_unsupported, "coupled stencil: lattice too large for one launch");
+          a.n_blocks = int(nblocks);
+          const unsigned int shared =
+            unsigned(2 * 3 * coupled_loads * coupled_threads * sizeof(number));
+          for (int s = 0; s < 3; ++s)
+            a.any_dmask |= a.op_dmask[s] | a.dst_dmask[s];
+          hipLaunchKernelGGL(coupled_stencil_kernel<number>, dim3(unsigned(nblocks)),
+                             dim3(coupled_threads), shared, stream, a);
+          dirichlet_faces(g, out);
+        }
     }
 
     /// Launches the one-pass generic kernel (cell_column_kernel in 3-D,
@@ -1383,10 +1542,32 @@ namespace ppf
       const prismspf::SolveBlock &blk = blocks[b];
       const GridDesc             &g   = *lf.grid;
       std::vector<int>            bf(blk.field_indices.begin(), blk.field_indices.end());
-      const SplitPlan            &plan = split_plan<number>(b, true).plan;
+      const PlanEntry            &entry = split_plan<number>(b, true);
+      const SplitPlan            &plan  = entry.plan;
       const bool                  use_split =
         path != OperatorPath::Generic && plan.eligible && plan.alpha_constant;
       const unsigned int nb = grid_for(g.n_nodes, block_size);
+      // Coupled components: the diagonal from the coefficients, once the plan has been
+      // checked against the generic path (an operator application on the fine lattice).
+      if constexpr (dim == 3 && degree == 2)
+        if (path == OperatorPath::Auto && generic_cell_block && entry.verified &&
+            takes_coupled(plan, g) &&
+            std::all_of(plan.coupled_slot, plan.coupled_slot + 3, [](int slot) {
+              return slot == prismspf::dependency_slot(prismspf::SRC);
+            }))
+          {
+            CoupledArgs<number> a = coupled_args<number>(g, plan, scaling);
+            for (std::size_t k = 0; k < bf.size(); ++k)
+              {
+                const int c = int(std::find(plan.coupled_out, plan.coupled_out + 3, bf[k]) -
+                                  plan.coupled_out);
+                hipLaunchKernelGGL(coupled_inverse_diagonal_kernel<number>, dim3(nb),
+                                   dim3(block_size), 0, stream, g, a, c,
+                                   inv_diag + int64_t(k) * g.n_nodes, scaling);
+              }
+            PPF_HIP_CHECK(hipGetLastError());
+            return;
+          }
       for (std::size_t k = 0; k < bf.size(); ++k)
         {
           const int f   = bf[k];
@@ -3808,6 +3989,7 @@ namespace ppf
     bool                                   explicit_fp32         = false;
     bool                                   explicit_fp32_copies  = false;
     std::set<int>                          explicit_mixed_noted;
+    std::set<std::pair<int, bool>>         coupled_noted;
     /// Consecutive explicit blocks in one launch (solve_explicit_pair): on/off (off by
     /// default: at 128^3 Q2 the fused launch takes 45 us against 2 x 13 us for the two
     /// stencil launches; its 5-wave workgroups hold 230 registers a lane, one
