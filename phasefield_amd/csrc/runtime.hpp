@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -202,7 +203,6 @@ namespace ppf
       fine = make_grid(inputs.spatial_discretization.global_refinement);
       PPF_HIP_CHECK(hipStreamCreate(&stream));
       reduce_buf.resize(2 * reduce_blocks + 8);
-      scalar_buf.resize(8);
       coarse_slots.resize(8);
       coarse_flag.resize(1);
       halt_flag.resize(max_pipeline_depth + 1);
@@ -597,16 +597,61 @@ namespace ppf
                          reduce_buf.get(), reduce_blocks);
     }
 
+    /// Sum of `count` partials of reduce_buf on the host, which polls for it.
     double
     finish_reduction(int count, int offset = 0)
     {
-      hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(reduce_threads), 0, stream,
-                         scalar_buf.get(), reduce_buf.get() + offset, count);
-      double r = 0.0;
-      PPF_HIP_CHECK(hipMemcpyAsync(&r, scalar_buf.get(), sizeof(double), hipMemcpyDeviceToHost,
-                                   stream));
-      sync();
-      return r;
+      const unsigned int tag = next_host_tag();
+      hipLaunchKernelGGL(reduce_to_host_kernel, dim3(1), dim3(reduce_threads), 0, stream,
+                         host_scalar(tag), reduce_buf.get() + offset, count, tag);
+      PPF_HIP_CHECK(hipGetLastError());
+      return wait_host_scalar(tag).first;
+    }
+
+    /// Tag of the next scalar sent to the host, and the ring entry it goes to: at most two
+    /// are under way at a time, so an entry is read before its next use.
+    unsigned int
+    next_host_tag()
+    {
+      host_tag = (host_tag + 1) & 0x7fffffffu;
+      return host_tag;
+    }
+
+    HostScalar *
+    host_scalar(unsigned int tag)
+    {
+      return host_scalars.get(host_scalar_ring) + tag % host_scalar_ring;
+    }
+
+    /// Waits for the scalar with this tag by polling its pinned entry (a copy and a stream
+    /// synchronization per scalar cost the GPU about 15 us); (value, flag).
+    std::pair<double, bool>
+    wait_host_scalar(unsigned int tag)
+    {
+      ++sync_count_;
+      const HostScalar *entry = host_scalar(tag);
+      const auto        ready = [&](unsigned int w) { return (w >> 1) == tag; };
+      const auto        word  = [&] {
+        return *reinterpret_cast<const volatile unsigned int *>(&entry->word);
+      };
+      unsigned int w = word();
+      for (unsigned long spin = 1; !ready(w); ++spin, w = word())
+        if (spin % 4096 == 0)
+          {
+            // Ends the wait if the stream has failed or drained without the scalar.
+            const hipError_t q = hipStreamQuery(stream);
+            if (q == hipSuccess)
+              {
+                w = word();
+                if (!ready(w))
+                  throw Error(status_internal, "scalar from the device missing");
+                break;
+              }
+            if (q != hipErrorNotReady)
+              PPF_HIP_CHECK(q);
+          }
+      std::atomic_thread_fence(std::memory_order_acquire);
+      return {*reinterpret_cast<const volatile double *>(&entry->value), (w & 1u) != 0};
     }
 
     // ------------------------------------------------------------ operator plans
@@ -2776,39 +2821,154 @@ namespace ppf
       unsigned int step   = 0;
       if (!(res <= tol))
         {
-          // The step scalars stay on the device: g.h alternates between slots 0 and 1,
-          // d.Ad is slot 2; alpha and beta are formed by the kernels that use them.  The
-          // host reads only the residual norm, once per step.
+          // The step scalars stay on the device: g.h alternates between slots 0 and 1;
+          // alpha and beta are formed by the kernels that use them.
           krylov_slots.resize(8);
-          double *ks = krylov_slots.get();
-          int     cur = 0;
-          precondition(b, ls.h.get(), ls.g.get());
-          axpby(ls.d.get(), -1.0, ls.h.get(), 0.0, n);
-          dot_to(ls.g.get(), ls.h.get(), n, ks + cur);
-          while (true)
-            {
-              ++step;
-              vmult_fine(b, ls.ad.get(), ls.d.get());
-              dot_to(ls.d.get(), ls.ad.get(), n, ks + 2);
-              hipLaunchKernelGGL(cg_update_slots_kernel, dim3(reduce_blocks),
-                                 dim3(reduce_threads), 0, stream, reduce_buf.get(), x,
-                                 ls.g.get(), ls.d.get(), ls.ad.get(), ks, cur, 2, n);
-              res = std::sqrt(finish_reduction(reduce_blocks));
-              if (!std::isfinite(res))
-                throw Error(status_nan, "linear solver produced a non-finite residual");
-              if (res <= tol || step >= max_steps)
-                break;
-              precondition(b, ls.h.get(), ls.g.get());
-              dot_to(ls.g.get(), ls.h.get(), n, ks + (1 - cur));
-              hipLaunchKernelGGL(cg_direction_slots_kernel, dim3(grid_for(n, 256)), dim3(256),
-                                 0, stream, ls.d.get(), ls.h.get(), ks, 1 - cur, cur, n);
-              cur = 1 - cur;
-            }
+          res = lin_params(b).preconditioner == prismspf::None
+                  ? cg_plain(b, x, tol, max_steps, step)
+                  : cg_preconditioned(b, x, tol, max_steps, step);
         }
       st.iterations     = int(step);
       st.final_residual = res;
       st.converged      = res <= tol ? 1 : 0;
       return st;
+    }
+
+    /// Sets the halt flag that operator launches carry for the life of the object.
+    struct HaltScope
+    {
+      HaltScope(Runtime &rt_, const int *flag)
+        : rt(rt_)
+        , before(rt_.enqueue_halt)
+      {
+        rt.enqueue_halt = flag;
+      }
+      ~HaltScope()
+      {
+        rt.enqueue_halt = before;
+      }
+      Runtime   &rt;
+      const int *before;
+    };
+
+    /// The CG loop without a preconditioner, from the residual in ls.g (see cg).  Steps are
+    /// enqueued one ahead of the residual the host reads: the step that meets the tolerance
+    /// sets a device flag that turns the launches behind it, the operator's included, into
+    /// no-ops, so the GPU never waits for the host and the result is that of the loop
+    /// that looks at every residual first.
+    double
+    cg_plain(int b, double *x, double tol, unsigned int max_steps, unsigned int &step)
+    {
+      LinearState       &ls = linear_state(b);
+      const int64_t      n  = ls.n;
+      const unsigned int nb = cg_grid(n);
+      double *ks = krylov_slots.get(), *dad = reduce_buf.get(), *gg = dad + reduce_blocks;
+      double *g = ls.g.get(), *d = ls.d.get();
+      if (cg_done.size() < 1)
+        cg_done.resize(1);
+      int *done = cg_done.get();
+      fill(done, 0, 1);
+      hipLaunchKernelGGL(cg_dot_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream, gg, g,
+                         g, n, (const int *) nullptr);
+      hipLaunchKernelGGL(cg_direction_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream,
+                         d, g, ks, 1, gg, int(nb), n, 1);
+      // (an enclosing halt flag keeps its meaning: no step is enqueued ahead under one)
+      const unsigned int ahead = enqueue_halt ? 0 : 1;
+      HaltScope          scope(*this, enqueue_halt ? enqueue_halt : done);
+      unsigned int       tags[2] = {};
+      const auto         enqueue = [&](unsigned int k) {
+        const int cur = int((k - 1) & 1u);
+        vmult_fine(b, ls.ad.get(), d);
+        hipLaunchKernelGGL(cg_dot_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream, dad,
+                           d, ls.ad.get(), n, done);
+        hipLaunchKernelGGL(cg_step_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream, gg,
+                           x, g, (double *) nullptr, d, ls.ad.get(), ks, cur, dad, int(nb), n,
+                           done);
+        tags[k & 1u] = next_host_tag();
+        hipLaunchKernelGGL(cg_turn_kernel, dim3(nb), dim3(reduce_threads), 0, stream, d, g, ks,
+                           cur, gg, int(nb), n, tol, done, host_scalar(tags[k & 1u]),
+                           tags[k & 1u]);
+        PPF_HIP_CHECK(hipGetLastError());
+      };
+      unsigned int enqueued = 0;
+      double       res      = 0.0;
+      while (true)
+        {
+          ++step;
+          while (enqueued < step || (enqueued < max_steps && enqueued < step + ahead))
+            enqueue(++enqueued);
+          const auto [value, end] = wait_host_scalar(tags[step & 1u]);
+          res                     = std::sqrt(value);
+          if (!std::isfinite(res))
+            throw Error(status_nan, "linear solver produced a non-finite residual");
+          if (end || step >= max_steps)
+            return res;
+        }
+    }
+
+    /// The CG loop with a preconditioner, from the residual in ls.g (see cg).  The host
+    /// reads every residual before it enqueues the preconditioner.  A multigrid V-cycle's
+    /// right-hand side is written by the step that computes the residual and its result is
+    /// read where it lies, in the levels' precision, instead of through FP64 copies.
+    double
+    cg_preconditioned(int b, double *x, double tol, unsigned int max_steps, unsigned int &step)
+    {
+      LinearState &ls = linear_state(b);
+      if (lin_params(b).preconditioner != prismspf::GMG)
+        return cg_loop<double>(b, x, tol, max_steps, step, nullptr, ls.h.get());
+      Level &top = ls.levels.back();
+      if (top.precision)
+        return cg_loop<float>(b, x, tol, max_steps, step, lvec<float>(top, 1),
+                              lvec<float>(top, 0));
+      return cg_loop<double>(b, x, tol, max_steps, step, lvec<double>(top, 1),
+                             lvec<double>(top, 0));
+    }
+
+    /// gt: the V-cycle's right-hand side (null: the Chebyshev preconditioner on the fine
+    /// level); h: the preconditioned residual.
+    template <typename T>
+    double
+    cg_loop(int b, double *x, double tol, unsigned int max_steps, unsigned int &step, T *gt,
+            const T *h)
+    {
+      LinearState       &ls = linear_state(b);
+      const int64_t      n  = ls.n;
+      const unsigned int nb = cg_grid(n);
+      double *ks = krylov_slots.get(), *part = reduce_buf.get(), *gg = part + reduce_blocks;
+      double *g = ls.g.get(), *d = ls.d.get();
+      const auto apply = [&] {
+        if (gt)
+          run_vcycle(b);
+        else
+          precondition(b, ls.h.get(), g);
+      };
+      const auto direction = [&](int cur, int first) {
+        hipLaunchKernelGGL(cg_dot_kernel<T>, dim3(nb), dim3(reduce_threads), 0, stream, part, g,
+                           h, n, (const int *) nullptr);
+        hipLaunchKernelGGL(cg_direction_kernel<T>, dim3(nb), dim3(reduce_threads), 0, stream, d,
+                           h, ks, cur, part, int(nb), n, first);
+      };
+      if (gt)
+        convert(gt, g, n);
+      apply();
+      direction(1, 1);
+      for (int cur = 0;; cur = 1 - cur)
+        {
+          ++step;
+          vmult_fine(b, ls.ad.get(), d);
+          hipLaunchKernelGGL(cg_dot_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream,
+                             part, d, ls.ad.get(), n, (const int *) nullptr);
+          hipLaunchKernelGGL(cg_step_kernel<T>, dim3(nb), dim3(reduce_threads), 0, stream, gg, x,
+                             g, gt, d, ls.ad.get(), ks, cur, part, int(nb), n,
+                             (const int *) nullptr);
+          const double res = std::sqrt(finish_reduction(int(nb), reduce_blocks));
+          if (!std::isfinite(res))
+            throw Error(status_nan, "linear solver produced a non-finite residual");
+          if (res <= tol || step >= max_steps)
+            return res;
+          apply();
+          direction(cur, 0);
+        }
     }
 
     // ------------------------------------------------------------ preconditioners
@@ -4022,7 +4182,11 @@ namespace ppf
     DeviceBuffer<double>                           zeros_d;
     DeviceBuffer<float>                            zeros_f;
     DeviceBuffer<double>                           reduce_buf;
-    DeviceBuffer<double>                           scalar_buf;
+    /// Scalars the host polls for (finish_reduction, cg).
+    static constexpr int                           host_scalar_ring = 4;
+    PinnedBuffer<HostScalar>                       host_scalars;
+    unsigned int                                   host_tag = 0;
+    DeviceBuffer<int>                              cg_done;
     DeviceBuffer<double>                           eig_slots;
     DeviceBuffer<double>                           coarse_slots;
     /// Coarse-grid solve handed to the next lhs stencil launch (coarse_cg_kernel).

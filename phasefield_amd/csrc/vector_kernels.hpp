@@ -8,6 +8,7 @@
 
 #include "grid.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace ppf
@@ -303,57 +304,163 @@ namespace ppf
       p[k] = 1.0 * z[k] + beta * p[k];
   }
 
-  /// CG update fused with the residual norm: x += alpha p, r += alpha Ap, partial |r|^2.
-  template <typename T>
-  __global__ void __launch_bounds__(reduce_threads)
-  cg_update_kernel(double *__restrict__ partial, T *__restrict__ x, T *__restrict__ r,
-                   const T *__restrict__ p, const T *__restrict__ ap, T alpha, int64_t n)
+  // ---------------------------------------------------------------- CG iteration
+  //
+  // A step is: operator application, d.Ad partial sums, cg_step_kernel, and either
+  // cg_turn_kernel (no preconditioner: h = g) or cg_residual_kernel, preconditioner, g.h
+  // partial sums and cg_direction_kernel.  No kernel only finishes a sum: every workgroup
+  // of the kernel that needs a dot product adds the few hundred partial sums itself, in one
+  // fixed order (8 kB from L2; a reduction kernel of its own costs a launch, about 5 us of
+  // a 45 us step at 140k nodes).  The residual norm goes to pinned host memory, which the
+  // host polls, so that no copy or stream synchronization ends a step.
+
+  /// Workgroups (and partial sums) of the kernels below for vectors of length n: enough to
+  /// stream long vectors, few partial sums for short ones.
+  inline unsigned int
+  cg_grid(int64_t n)
+  {
+    return unsigned(std::min<int64_t>(std::max<int64_t>((n + 1023) / 1024, 1), reduce_blocks));
+  }
+
+  /// Sum of one double per thread in every thread of the block.
+  __device__ PPF_INLINE double
+  block_total(double v)
+  {
+    __shared__ double total;
+    v = block_sum(v);
+    if (threadIdx.x == 0)
+      total = v;
+    __syncthreads();
+    v = total;
+    __syncthreads();
+    return v;
+  }
+
+  /// Sum of `count` partial sums, the same bits in every thread of every block.
+  __device__ PPF_INLINE double
+  sum_partials(const double *__restrict__ partial, int count)
   {
     double s = 0.0;
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * blockDim.x)
-      {
-        x[i] += alpha * p[i];
-        const T ri = r[i] + alpha * ap[i];
-        r[i]       = ri;
-        s += double(ri) * double(ri);
-      }
+    for (int i = threadIdx.x; i < count; i += reduce_threads)
+      s += partial[i];
+    return block_total(s);
+  }
+
+  /// A scalar for the polling host: value, then (tag << 1) | flag once it is visible.
+  struct HostScalar
+  {
+    double       value;
+    unsigned int word;
+  };
+
+  __device__ PPF_INLINE void
+  tell_host(HostScalar *to, double value, unsigned int tag, bool flag)
+  {
+    *reinterpret_cast<volatile double *>(&to->value) = value;
+    __threadfence_system();
+    *reinterpret_cast<volatile unsigned int *>(&to->word) = (tag << 1) | (flag ? 1u : 0u);
+  }
+
+  /// Sums `count` partials and tells the host.
+  __global__ void __launch_bounds__(reduce_threads)
+  reduce_to_host_kernel(HostScalar *to, const double *__restrict__ partial, int count,
+                        unsigned int tag)
+  {
+    const double s = sum_partials(partial, count);
+    if (threadIdx.x == 0)
+      tell_host(to, s, tag, false);
+  }
+
+  /// Per-block partial sums of x.y; nothing once *done is set (done may be null).
+  template <typename T>
+  __global__ void __launch_bounds__(reduce_threads)
+  cg_dot_kernel(double *__restrict__ partial, const double *__restrict__ x,
+                const T *__restrict__ y, int64_t n, const int *done)
+  {
+    if (done && *done)
+      return;
+    double s = 0.0;
+    for (int64_t i = int64_t(blockIdx.x) * reduce_threads + threadIdx.x; i < n;
+         i += int64_t(gridDim.x) * reduce_threads)
+      s += x[i] * double(y[i]);
     s = block_sum(s);
     if (threadIdx.x == 0)
       partial[blockIdx.x] = s;
   }
 
-  /// p = -h + beta p
+  /// x += alpha d, g += alpha Ad with alpha = s[cur] / (d.Ad), and partial sums of g.g; the
+  /// new g also goes to `gt` (the preconditioner's copy, in its precision) unless null.
   template <typename T>
-  __global__ void
-  cg_direction_kernel(T *__restrict__ p, const T *__restrict__ h, T beta, int64_t n)
-  {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n)
-      p[i] = -h[i] + beta * p[i];
-  }
-
-  /// cg_update_kernel with alpha = s[num] / s[den] read from device slots (the same
-  /// double division the host would do).
   __global__ void __launch_bounds__(reduce_threads)
-  cg_update_slots_kernel(double *__restrict__ partial, double *__restrict__ x,
-                         double *__restrict__ r, const double *__restrict__ p,
-                         const double *__restrict__ ap, const double *__restrict__ s, int num,
-                         int den, int64_t n)
+  cg_step_kernel(double *__restrict__ partial_gg, double *__restrict__ x,
+                 double *__restrict__ g, T *__restrict__ gt, const double *__restrict__ d,
+                 const double *__restrict__ ad, const double *__restrict__ s, int cur,
+                 const double *__restrict__ partial_dad, int count, int64_t n, const int *done)
   {
-    const double alpha = s[num] / s[den];
+    if (done && *done)
+      return;
+    const double alpha = s[cur] / sum_partials(partial_dad, count);
     double       acc   = 0.0;
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * blockDim.x)
+    for (int64_t i = int64_t(blockIdx.x) * reduce_threads + threadIdx.x; i < n;
+         i += int64_t(gridDim.x) * reduce_threads)
       {
-        x[i] += alpha * p[i];
-        const double ri = r[i] + alpha * ap[i];
-        r[i]            = ri;
-        acc += ri * ri;
+        x[i] += alpha * d[i];
+        const double gi = g[i] + alpha * ad[i];
+        g[i]            = gi;
+        if (gt)
+          gt[i] = T(gi);
+        acc += gi * gi;
       }
     acc = block_sum(acc);
     if (threadIdx.x == 0)
-      partial[blockIdx.x] = acc;
+      partial_gg[blockIdx.x] = acc;
+  }
+
+  /// Unpreconditioned end of a step: gg = g.g (also the next g.h); if |g| <= tol (or it is
+  /// not a number) *done is set and d stays, else d = -g + (gg / s[cur]) d and s[1 - cur] =
+  /// gg.  Tells the host gg and whether the iteration is done.
+  __global__ void __launch_bounds__(reduce_threads)
+  cg_turn_kernel(double *__restrict__ d, const double *__restrict__ g, double *__restrict__ s,
+                 int cur, const double *__restrict__ partial_gg, int count, int64_t n,
+                 double tol, int *done, HostScalar *to, unsigned int tag)
+  {
+    if (*done)
+      return;
+    const double gg  = sum_partials(partial_gg, count);
+    const bool   end = !(std::sqrt(gg) > tol);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+      {
+        tell_host(to, gg, tag, end);
+        // A block of this launch that starts after this store leaves at once, as it would
+        // have by `end`.
+        if (end)
+          *done = 1;
+      }
+    if (end)
+      return;
+    const double beta = gg / s[cur];
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+      s[1 - cur] = gg;
+    for (int64_t i = int64_t(blockIdx.x) * reduce_threads + threadIdx.x; i < n;
+         i += int64_t(gridDim.x) * reduce_threads)
+      d[i] = -g[i] + beta * d[i];
+  }
+
+  /// d = -h + beta d with beta = (g.h) / s[cur] from the partial sums of g.h, which becomes
+  /// s[1 - cur]; with `first` set d = -h.
+  template <typename T>
+  __global__ void __launch_bounds__(reduce_threads)
+  cg_direction_kernel(double *__restrict__ d, const T *__restrict__ h, double *__restrict__ s,
+                      int cur, const double *__restrict__ partial_gh, int count, int64_t n,
+                      int first)
+  {
+    const double gh   = sum_partials(partial_gh, count);
+    const double beta = first ? 0.0 : gh / s[cur];
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+      s[1 - cur] = gh;
+    for (int64_t i = int64_t(blockIdx.x) * reduce_threads + threadIdx.x; i < n;
+         i += int64_t(gridDim.x) * reduce_threads)
+      d[i] = first ? -double(h[i]) : -double(h[i]) + beta * d[i];
   }
 
   /// BiCGStab scalars in device slots: 0 rho, 1 alpha, 2 omega, 3 r.rbar, 4 rbar.v,
@@ -422,16 +529,6 @@ namespace ppf
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n)
       x[i] += s[1] * y[i] + s[2] * z[i];
-  }
-
-  /// cg_direction_kernel with beta = s[num] / s[den] read from device slots.
-  __global__ void
-  cg_direction_slots_kernel(double *__restrict__ p, const double *__restrict__ h,
-                            const double *__restrict__ s, int num, int den, int64_t n)
-  {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n)
-      p[i] = -h[i] + (s[num] / s[den]) * p[i];
   }
 
   /// First Chebyshev step from x = 0 (A x = 0): d = c2 P^{-1} b, x = d.  Same values as
