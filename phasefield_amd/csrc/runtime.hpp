@@ -1298,12 +1298,6 @@ namespace ppf
     launch_stencil(int b, bool lhs, const GridDesc &g, const DepTable<ST> &deps,
                    const OutTable<ST> &out, const SplitPlan &plan)
     {
-      // Small lattices (multigrid's coarse levels) go to the one-thread-per-node kernel:
-      // a tile's march over its z planes would take longer than the whole lattice node
-      // by node.  The fused coarse solve rides on this launch and keeps it.
-      if (g.n_nodes < stencil_min_nodes && !coarse_pending &&
-          !(probe_req.pending && probe_req.block == b))
-        return false;
       StencilArgs<number, ST> a {};
       // Distinct (field, slot) operands of the gradient terms.
       int op_field[stencil_max_ops], op_slot[stencil_max_ops];
@@ -1331,6 +1325,10 @@ namespace ppf
             }
           a.beta[tm.out_field][k] += number(tm.beta);
         }
+      // Two operands on a small lattice: node by node (split_operator_kernel).
+      if (a.n_ops > 1 && g.n_nodes < stencil_min_nodes && !coarse_pending &&
+          !(probe_req.pending && probe_req.block == b))
+        return false;
       // Unused operand and value entries point at an array of the lattice size so the
       // kernel loads them without a branch (their values are never used).
       const ST *any_array = nullptr;
@@ -1453,6 +1451,61 @@ namespace ppf
             return true;
           }
 
+      const auto &pde = *pde_of<number>();
+      // The increment's NaN probe rides on this launch if it is the block's last kernel
+      // (no Dirichlet-value faces kernel follows).
+      bool faces_follow = false;
+      if (out.dirichlet_write == dirichlet_value)
+        for (int f = 0; f < PPF_MAX_FIELDS; ++f)
+          faces_follow = faces_follow || ((out.out_mask & (1u << f)) && out.dirichlet_mask[f]);
+      const auto take_probe = [&] {
+        if constexpr (std::is_same_v<ST, double>)
+          if (probe_req.pending && probe_req.block == b && !faces_follow)
+            {
+              a.probe_result = probe_req.result;
+              a.probe_halt   = probe_req.halt;
+              a.probe_hmask  = probe_req.hmask;
+              a.probe_tag    = probe_req.tag;
+              a.probe_n      = probe_req.fields.n;
+              for (int f = 0; f < PPF_MAX_FIELDS; ++f)
+                a.probe_ptr[f] = probe_req.fields.ptr[f];
+              probe_req.pending = false;
+              probe_req.taken   = true;
+            }
+      };
+      using I1 = std::integral_constant<int, 1>;
+      using I2 = std::integral_constant<int, 2>;
+      using I4 = std::integral_constant<int, 4>;
+      using I8 = std::integral_constant<int, 8>;
+
+      // Lattices below stencil_min_nodes: column by column instead of by marching tiles.
+      if (a.n_ops <= 1 && g.n_nodes < stencil_min_nodes)
+        {
+          const auto go = [&](auto masked_c) {
+            constexpr bool MK = decltype(masked_c)::value;
+            constexpr int  ZC = stencil_column_planes<dim>;
+            a.tiles_x  = int(grid_for(int64_t(a.n[0]) * a.n[1], stencil_column_threads));
+            a.chunks_z = (a.n[2] + ZC - 1) / ZC;
+            const int64_t nblocks = int64_t(a.tiles_x) * a.chunks_z;
+            if (nblocks >= (int64_t(1) << 31))
+              return false;
+            a.n_blocks = int(nblocks);
+            take_probe();
+            const dim3 grid {unsigned(nblocks)}, threads {stencil_column_threads};
+            if (lhs)
+              hipLaunchKernelGGL(
+                (stencil_column_kernel<PDE<number>, dim, degree, number, true, id, App::n_fields, MK, ST>),
+                grid, threads, 0, stream, pde, a, out, timer);
+            else
+              hipLaunchKernelGGL(
+                (stencil_column_kernel<PDE<number>, dim, degree, number, false, id, App::n_fields, MK, ST>),
+                grid, threads, 0, stream, pde, a, out, timer);
+            dirichlet_faces(g, out);
+            return true;
+          };
+          return a.any_dmask != 0 ? go(std::true_type {}) : go(std::false_type {});
+        }
+
       // Tile shape: waves per workgroup x rows per wave.  Default 4 x 2 (measured
       // faster than 4 x 4 at 129^3 and 257^3: fewer registers); two staged operands
       // take 4 x 2 or 8 x 1 (more rows would spill in FP64).
@@ -1517,26 +1570,8 @@ namespace ppf
         return false;
       a.n_blocks = int(nblocks);
 
-      const auto &pde = *pde_of<number>();
-      // The increment's NaN probe rides on this launch if it is the block's last kernel
-      // (no Dirichlet-value faces kernel follows) and node 0 lies in tile 0.
-      bool faces_follow = false;
-      if (out.dirichlet_write == dirichlet_value)
-        for (int f = 0; f < PPF_MAX_FIELDS; ++f)
-          faces_follow = faces_follow || ((out.out_mask & (1u << f)) && out.dirichlet_mask[f]);
-      if constexpr (std::is_same_v<ST, double>)
-        if (probe_req.pending && probe_req.block == b && !faces_follow && a.n_blocks > 0)
-          {
-            a.probe_result = probe_req.result;
-            a.probe_halt   = probe_req.halt;
-            a.probe_hmask  = probe_req.hmask;
-            a.probe_tag    = probe_req.tag;
-            a.probe_n      = probe_req.fields.n;
-            for (int f = 0; f < PPF_MAX_FIELDS; ++f)
-              a.probe_ptr[f] = probe_req.fields.ptr[f];
-            probe_req.pending = false;
-            probe_req.taken   = true;
-          }
+      if (a.n_blocks > 0) // node 0 lies in tile 0
+        take_probe();
       const dim3  grid(unsigned(nblocks + nrem)), threads(stencil_tx, unsigned(waves));
       auto        go = [&](auto waves_c, auto rows_c, auto ops_c) {
         constexpr int WV = decltype(waves_c)::value;
@@ -1551,10 +1586,6 @@ namespace ppf
             (stencil_operator_kernel<PDE<number>, dim, degree, number, false, id, App::n_fields, WV, RR, NS, ST>),
             grid, threads, 0, stream, pde, a, out, timer);
       };
-      using I1 = std::integral_constant<int, 1>;
-      using I2 = std::integral_constant<int, 2>;
-      using I4 = std::integral_constant<int, 4>;
-      using I8 = std::integral_constant<int, 8>;
       if (a.n_ops > 1)
         {
           if (waves == 8)

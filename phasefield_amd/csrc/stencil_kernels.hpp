@@ -743,6 +743,204 @@ namespace ppf
       run(std::integral_constant<bool, false> {});
   }
 
+  /// Planes a thread of stencil_column_kernel owns.
+  template <int dim>
+  constexpr int stencil_column_planes = dim == 3 ? 4 : 1;
+  constexpr int stencil_column_threads = 256;
+
+  /// The same operator, with at most one stencil operand, without tiles: a thread owns one (x, y) column of a few planes, the
+  /// threads of a workgroup consecutive nodes of the flattened x-y plane (no lane is idle
+  /// at a ragged width).  Every operand value comes from the caches through a load of its
+  /// own, all of them issued before the first is used: there is no march, so the time of a
+  /// launch is about one memory latency plus the issue of 9 (Q1: 6) loads per node, where
+  /// a tile of stencil_operator_kernel waits once per plane.  Same arithmetic, same bits.
+  ///
+  /// a.tiles_x: workgroups per plane, a.chunks_z: plane groups, a.n_blocks: their product.
+  /// MASKED: some operand, input or output has Dirichlet faces.
+  template <class PDE, int dim, int degree, typename number, bool lhs, int block_id, int NF,
+            bool MASKED, typename ST = number>
+  __global__ void __launch_bounds__(stencil_column_threads)
+  stencil_column_kernel(const PDE pde, const StencilArgs<number, ST> a, const OutTable<ST> out,
+                        const prismspf::SimulationTimer timer)
+  {
+    constexpr int RAD = degree;
+    constexpr int ZC  = stencil_column_planes<dim>;
+    static_assert(dim != 3 || degree != 2 || ZC % 2 == 0, "z parity from the plane index");
+    if (halted(out.halt))
+      return;
+    const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2];
+    const int p0 = a.periodic[0], p1 = a.periodic[1], p2 = a.periodic[2];
+    // Consecutive workgroups of a plane group on one XCD (see stencil_operator_kernel).
+    const int q8  = a.n_blocks / 8;
+    const int b   = blockIdx.x;
+    const int lb  = b < 8 * q8 ? (b % 8) * q8 + b / 8 : b;
+    const int chk = lb / a.tiles_x;
+    const unsigned int q =
+      unsigned(lb - chk * a.tiles_x) * stencil_column_threads + threadIdx.x;
+    if (q >= unsigned(n0) * unsigned(n1))
+      return;
+    const int          y  = int(q / unsigned(n0));
+    const int          x  = int(q - unsigned(y) * unsigned(n0));
+    const int          z0 = chk * ZC;
+    const unsigned int plane_bytes = unsigned(n0) * unsigned(n1) * unsigned(sizeof(ST));
+    const unsigned int own         = q * unsigned(sizeof(ST));
+
+    // In-plane neighbours (byte offsets and, where a face matters, face bits).
+    unsigned int xo[2 * RAD], yo[2 * RAD], xf[2 * RAD], yf[2 * RAD];
+    const unsigned int fbx = face_bits(x, n0, p0, 0), fby = face_bits(y, n1, p1, 1);
+#pragma unroll
+    for (int k = 0; k < 2 * RAD; ++k)
+      {
+        const int o  = k < RAD ? k - RAD : k - RAD + 1; // -RAD .. -1, 1 .. RAD
+        const int xs = source_coord(x + o, n0, p0), ys = source_coord(y + o, n1, p1);
+        xo[k] = own + unsigned(xs - x) * unsigned(sizeof(ST));
+        yo[k] = own + unsigned((ys - y) * n0) * unsigned(sizeof(ST));
+        xf[k] = face_bits(xs, n0, p0, 0) | fby;
+        yf[k] = face_bits(ys, n1, p1, 1) | fbx;
+      }
+    const auto source_z = [&](int z) {
+      return unsigned(z) < unsigned(n2) ? z : source_coord(z, n2, p2);
+    };
+
+    const buffer_rsrc r_op = make_rsrc(a.op[0]);
+    buffer_rsrc       r_dst[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      r_dst[f] = make_rsrc(out.dst[f]);
+
+    // Every load first.
+    ST column[ZC + 2 * RAD], xn[ZC][2 * RAD], yn[ZC][2 * RAD];
+    ST value[ZC][NF][PPF_N_SLOTS];
+    if constexpr (dim == 3)
+      {
+#pragma unroll
+        for (int k = 0; k < ZC + 2 * RAD; ++k)
+          column[k] =
+            buffer_load<ST>(r_op, own, unsigned(source_z(z0 - RAD + k)) * plane_bytes);
+      }
+    else
+      column[RAD] = buffer_load<ST>(r_op, own, 0);
+#pragma unroll
+    for (int k = 0; k < ZC; ++k)
+      {
+        const unsigned int po = dim == 3 ? unsigned(min(z0 + k, n2 - 1)) * plane_bytes : 0u;
+#pragma unroll
+        for (int o = 0; o < 2 * RAD; ++o)
+          {
+            xn[k][o] = buffer_load<ST>(r_op, xo[o], po);
+            yn[k][o] = buffer_load<ST>(r_op, yo[o], po);
+          }
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+          for (int s = 0; s < PPF_N_SLOTS; ++s)
+            value[k][f][s] = buffer_load<ST>(make_rsrc(a.val[f][s]), own, po);
+      }
+
+    // Taps and scale factors of the column.
+    const bool   xodd = degree == 2 && (x & 1), yodd = degree == 2 && (y & 1);
+    number       wx[RAD + 1], wy[RAD + 1];
+#pragma unroll
+    for (int o = 0; o <= RAD; ++o)
+      {
+        wx[o] = xodd ? a.tap[0][1][o] : a.tap[0][0][o];
+        wy[o] = yodd ? a.tap[1][1][o] : a.tap[1][0][o];
+      }
+    const int    cx = scale_class<degree>(x, n0, p0), cy = scale_class<degree>(y, n1, p1);
+    const number sx = cx == 0 ? a.sfac[0][0] : (cx == 1 ? a.sfac[0][1] : a.sfac[0][2]);
+    const number sy = cy == 0 ? a.sfac[1][0] : (cy == 1 ? a.sfac[1][1] : a.sfac[1][2]);
+
+#pragma unroll
+    for (int k = 0; k < ZC; ++k)
+      {
+        const int z = z0 + k;
+        if (dim == 3 && z >= n2)
+          break;
+        const unsigned int po  = dim == 3 ? unsigned(z) * plane_bytes : 0u;
+        const unsigned int fbz = face_bits(z, n2, p2, 2);
+        constexpr bool     q2  = degree == 2;
+        const bool         zodd = q2 && (k & 1); // z0 is even
+        number             wz[RAD + 1], sz = number(1);
+#pragma unroll
+        for (int o = 0; o <= RAD; ++o)
+          wz[o] = dim == 3 ? (zodd ? a.tap[2][1][o] : a.tap[2][0][o]) : number(0);
+        if constexpr (dim == 3)
+          sz = (!p2 && (z == 0 || z == n2 - 1)) ? a.sfac[2][2]
+                                                 : (zodd ? a.sfac[2][0] : a.sfac[2][1]);
+
+        const unsigned int dm   = MASKED ? a.op_dmask[0] : 0u;
+        const auto         keep = [&](ST v, unsigned int fb) {
+          return MASKED && (fb & dm) ? number(0) : number(v);
+        };
+        const auto line = [&](int o) { // column value at z + o
+          return keep(column[k + RAD + o],
+                      fbx | fby | (MASKED ? face_bits(source_z(z + o), n2, p2, 2) : 0u));
+        };
+        const number centre = keep(column[dim == 3 ? k + RAD : RAD], fbx | fby | fbz);
+        number       lap    = (wx[0] + (wy[0] + wz[0])) * centre;
+#pragma unroll
+        for (int o = 1; o <= RAD; ++o)
+          {
+            lap = fma(wx[o],
+                      keep(xn[k][RAD - o], xf[RAD - o] | fbz) +
+                        keep(xn[k][RAD + o - 1], xf[RAD + o - 1] | fbz),
+                      lap);
+            lap = fma(wy[o],
+                      keep(yn[k][RAD - o], yf[RAD - o] | fbz) +
+                        keep(yn[k][RAD + o - 1], yf[RAD + o - 1] | fbz),
+                      lap);
+            if constexpr (dim == 3)
+              lap = fma(wz[o], line(-o) + line(o), lap);
+          }
+
+        const unsigned int                            fb = fbx | fby | fbz;
+        prismspf::FieldContainer<dim, degree, number> fc;
+        fc.q_point[0] = number(a.q_lower[0] + x * a.q_step[0]);
+        fc.q_point[1] = number(a.q_lower[1] + y * a.q_step[1]);
+        if constexpr (dim == 3)
+          fc.q_point[2] = number(a.q_lower[2] + z * a.q_step[2]);
+        fc.element_volume = number(a.element_volume);
+#pragma unroll
+        for (int f = 0; f < PPF_MAX_FIELDS; ++f)
+#pragma unroll
+          for (int s = 0; s < PPF_N_SLOTS; ++s)
+            {
+              number v = number(0);
+              if (f < NF)
+                {
+                  const int fi = f < NF ? f : 0;
+                  const int al = a.val_alias[fi][s];
+                  v            = number(value[k][fi][s]);
+                  if (MASKED && (fb & a.val_dmask[fi][s]))
+                    v = number(0);
+                  if (al == 0)
+                    v = centre;
+                }
+              fc.value[f][s] = v;
+#pragma unroll
+              for (int d = 0; d < dim; ++d)
+                fc.gradient[f][s][d] = number(0);
+            }
+        fc.clear_terms();
+        call_hook<PDE, dim, degree, number, lhs, block_id>(pde, fc, timer);
+
+        const number scale = sx * (sy * sz);
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          {
+            if (!(out.out_mask & (1u << f)))
+              continue;
+            number acc = (fc.value_term_mask & (1u << f)) ? fc.value_term[f] : number(0);
+            acc = fma(a.beta[f][0], lap, acc);
+            const bool dir = MASKED && (fb & out.dirichlet_mask[f]) != 0;
+            if (!(dir && out.dirichlet_write == dirichlet_value))
+              buffer_store(dir ? ST(0) : ST(scale * acc), r_dst[f], own, po, a.nt_store != 0);
+          }
+        if (k == 0 && a.probe_result && chk == 0 && q == 0)
+          stencil_probe(a);
+      }
+  }
+
   /// Vectors and limits of a coarse-grid CG run by one workgroup.
   struct CoarseCgArgs
   {
