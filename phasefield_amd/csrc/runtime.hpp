@@ -2170,8 +2170,6 @@ namespace ppf
       bool                                eigenvalues_estimated = false;
       std::vector<DeviceBuffer<double>>   field_d[PPF_MAX_FIELDS];
       std::vector<DeviceBuffer<float>>    field_f[PPF_MAX_FIELDS];
-      DeviceBuffer<double>                tmp_d[2]; // separable transfers to the coarser level
-      DeviceBuffer<float>                 tmp_f[2];
     };
 
     struct LinearState
@@ -3581,109 +3579,54 @@ namespace ppf
       for (std::size_t k = 0; k < blocks[b].field_indices.size(); ++k)
         {
           const int f = int(*std::next(blocks[b].field_indices.begin(), k));
-          restrict_separable<T>(lvec<T>(c, 1) + k * c.grid.n_nodes, c.grid,
-                                lvec<T>(l, 2) + k * l.grid.n_nodes, l, dirichlet_mask(f));
+          restrict_to<T>(lvec<T>(c, 1) + k * c.grid.n_nodes, c.grid,
+                         lvec<T>(l, 2) + k * l.grid.n_nodes, l.grid, dirichlet_mask(f));
         }
       v_cycle<T>(b, li - 1);
       for (std::size_t k = 0; k < blocks[b].field_indices.size(); ++k)
         {
           const int f = int(*std::next(blocks[b].field_indices.begin(), k));
-          prolongate_add_separable<T>(lvec<T>(l, 0) + k * l.grid.n_nodes, l,
-                                      lvec<T>(c, 0) + k * c.grid.n_nodes, c.grid,
-                                      dirichlet_mask(f));
+          prolongate_add<T>(lvec<T>(l, 0) + k * l.grid.n_nodes, l.grid,
+                            lvec<T>(c, 0) + k * c.grid.n_nodes, c.grid, dirichlet_mask(f));
         }
       chebyshev<T>(A, linv<T>(l), n, deg, l.lambda_max, l.lambda_min, lvec<T>(l, 0),
                    lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), false, tab);
     }
 
-    /// Scratch lattices of the separable transfers between level l and the next
-    /// coarser one: [0] coarse x-extent by the fine y, z extents; [1] coarse x, y by fine z.
-    template <typename T>
-    T *
-    transfer_tmp(Level &l, int i, int64_t n)
-    {
-      auto &buf = [&]() -> auto & {
-        if constexpr (std::is_same_v<T, float>)
-          return l.tmp_f[i];
-        else
-          return l.tmp_d[i];
-      }();
-      if (buf.size() < n)
-        buf.resize(n);
-      return buf.get();
-    }
-
-    /// fine += P coarse (fine Dirichlet nodes untouched), one pass per axis.
-    template <typename T>
-    void
-    prolongate_add_separable(T *fine_v, Level &l, const T *coarse_v, const GridDesc &gc,
-                             unsigned int mask)
-    {
-      const GridDesc &gf = l.grid;
-      const int c0 = gc.nodes[0], c1 = gc.nodes[1], c2 = gc.nodes[2];
-      const int f0 = gf.nodes[0], f1 = gf.nodes[1], f2 = gf.nodes[2];
-      const T  *in = coarse_v;
-      if constexpr (dim == 3)
-        {
-          // z: (c0, c1, c2) -> (c0, c1, f2)
-          T *t1 = transfer_tmp<T>(l, 1, int64_t(c0) * c1 * f2);
-          hipLaunchKernelGGL((transfer_axis_kernel<dim, degree, T, false, 0, 2>),
-                             transfer_grid(c0, c1, f2), dim3(256), 0, stream, t1, in, c0, c1,
-                             c0, c1, gc, gf, 0u);
-          in = t1;
-        }
-      // y: (c0, c1, f2) -> (c0, f1, f2)
-      T *t0 = transfer_tmp<T>(l, 0, int64_t(c0) * f1 * f2);
-      hipLaunchKernelGGL((transfer_axis_kernel<dim, degree, T, false, 0, 1>),
-                         transfer_grid(c0, f1, f2), dim3(256), 0, stream, t0, in, c0, f1, c0,
-                         c1, gc, gf, 0u);
-      // x: (c0, f1, f2) -> fine, added
-      hipLaunchKernelGGL((transfer_axis_kernel<dim, degree, T, false, 1, 0>),
-                         transfer_grid(f0, f1, f2), dim3(256), 0, stream, fine_v, t0, f0, f1,
-                         c0, f1, gc, gf, mask);
-    }
-
-    /// Launch grid of transfer_axis_kernel for an e0 x e1 x e2 output lattice.
+    /// Launch grid of a transfer kernel: a plane of e0 x e1 nodes, `groups` groups of planes.
     static dim3
-    transfer_grid(int e0, int e1, int e2)
+    transfer_grid(int e0, int e1, int groups)
     {
       const int64_t plane = int64_t(e0) * e1;
-      if (plane >= (int64_t(1) << 31) || e2 > 65535)
+      if (plane >= (int64_t(1) << 31) || groups > 65535)
         throw Error(status_unsupported, "transfer: lattice too large for one launch");
-      return dim3(grid_for(plane, 256), unsigned(e2));
+      return dim3(grid_for(plane, transfer_threads), unsigned(groups));
     }
 
-    /// coarse = P^T fine (coarse Dirichlet nodes zero), one pass per axis.
+    /// fine += P coarse (fine Dirichlet nodes untouched).
     template <typename T>
     void
-    restrict_separable(T *coarse_v, const GridDesc &gc, const T *fine_v, Level &l,
-                       unsigned int mask)
+    prolongate_add(T *fine_v, const GridDesc &gf, const T *coarse_v, const GridDesc &gc,
+                   unsigned int mask)
     {
-      const GridDesc &gf = l.grid;
-      const int c0 = gc.nodes[0], c1 = gc.nodes[1], c2 = gc.nodes[2];
-      const int f0 = gf.nodes[0], f1 = gf.nodes[1], f2 = gf.nodes[2];
-      // x: (f0, f1, f2) -> (c0, f1, f2)
-      T *t0 = transfer_tmp<T>(l, 0, int64_t(c0) * f1 * f2);
-      hipLaunchKernelGGL((transfer_axis_kernel<dim, degree, T, true, 0, 0>),
-                         transfer_grid(c0, f1, f2), dim3(256), 0, stream, t0, fine_v, c0, f1,
-                         f0, f1, gf, gc, 0u);
-      if constexpr (dim == 3)
-        {
-          // y: (c0, f1, f2) -> (c0, c1, f2)
-          T *t1 = transfer_tmp<T>(l, 1, int64_t(c0) * c1 * f2);
-          hipLaunchKernelGGL((transfer_axis_kernel<dim, degree, T, true, 0, 1>),
-                             transfer_grid(c0, c1, f2), dim3(256), 0, stream, t1, t0, c0, c1,
-                             c0, f1, gf, gc, 0u);
-          // z: (c0, c1, f2) -> coarse, Dirichlet nodes zero
-          hipLaunchKernelGGL((transfer_axis_kernel<dim, degree, T, true, 2, 2>),
-                             transfer_grid(c0, c1, c2), dim3(256), 0, stream, coarse_v, t1,
-                             c0, c1, c0, c1, gf, gc, mask);
-        }
-      else
-        // y: (c0, f1) -> coarse, Dirichlet nodes zero
-        hipLaunchKernelGGL((transfer_axis_kernel<dim, degree, T, true, 2, 1>),
-                             transfer_grid(c0, c1, c2), dim3(256), 0, stream, coarse_v, t0,
-                             c0, c1, c0, f1, gf, gc, mask);
+      const int zc     = 2 * degree;
+      const int layers = dim == 3 ? (gf.nodes[2] + zc - 1) / zc : 1;
+      hipLaunchKernelGGL((prolongate_add_kernel<dim, degree, T>),
+                         transfer_grid(gf.nodes[0], gf.nodes[1], layers), dim3(transfer_threads),
+                         0, stream, fine_v, coarse_v, gc, gf, mask);
+    }
+
+    /// coarse = P^T fine (coarse Dirichlet nodes zero).
+    template <typename T>
+    void
+    restrict_to(T *coarse_v, const GridDesc &gc, const T *fine_v, const GridDesc &gf,
+                unsigned int mask)
+    {
+      constexpr int zc     = restrict_planes<dim>;
+      const int     groups = dim == 3 ? (gc.nodes[2] + zc - 1) / zc : 1;
+      hipLaunchKernelGGL((restrict_kernel<dim, degree, T>),
+                         transfer_grid(gc.nodes[0], gc.nodes[1], groups), dim3(transfer_threads),
+                         0, stream, coarse_v, fine_v, gc, gf, mask);
     }
 
     template <typename T>
