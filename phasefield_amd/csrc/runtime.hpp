@@ -1492,14 +1492,31 @@ namespace ppf
             a.n_blocks = int(nblocks);
             take_probe();
             const dim3 grid {unsigned(nblocks)}, threads {stencil_column_threads};
+            // A smoother waiting for A x takes the launch (see smoother_step).
+            if constexpr (std::is_same_v<number, ST>)
+              if (lhs && smoother_request<ST>().pending)
+                {
+                  auto &req   = smoother_request<ST>();
+                  req.pending = false;
+                  if (req.kind == Smoother::Chebyshev)
+                    hipLaunchKernelGGL(
+                      (stencil_column_kernel<PDE<number>, dim, degree, number, true, id, App::n_fields, MK, ST, Smoother::Chebyshev>),
+                      grid, threads, 0, stream, pde, a, out, timer, req.args);
+                  else
+                    hipLaunchKernelGGL(
+                      (stencil_column_kernel<PDE<number>, dim, degree, number, true, id, App::n_fields, MK, ST, Smoother::Residual>),
+                      grid, threads, 0, stream, pde, a, out, timer, req.args);
+                  return true;
+                }
+            const SmootherArgs<ST> no_smoother {};
             if (lhs)
               hipLaunchKernelGGL(
                 (stencil_column_kernel<PDE<number>, dim, degree, number, true, id, App::n_fields, MK, ST>),
-                grid, threads, 0, stream, pde, a, out, timer);
+                grid, threads, 0, stream, pde, a, out, timer, no_smoother);
             else
               hipLaunchKernelGGL(
                 (stencil_column_kernel<PDE<number>, dim, degree, number, false, id, App::n_fields, MK, ST>),
-                grid, threads, 0, stream, pde, a, out, timer);
+                grid, threads, 0, stream, pde, a, out, timer, no_smoother);
             dirichlet_faces(g, out);
             return true;
           };
@@ -3187,16 +3204,76 @@ namespace ppf
                   unsigned(g.n_fields));
     }
 
+    /// A smoother step (Chebyshev update or residual) waiting for the operator application
+    /// that forms its A x.
+    template <typename T>
+    struct SmootherRequest
+    {
+      bool            pending = false;
+      Smoother        kind    = Smoother::None;
+      SmootherArgs<T> args {};
+    };
+
+    template <typename T>
+    SmootherRequest<T> &
+    smoother_request()
+    {
+      if constexpr (std::is_same_v<T, float>)
+        return smoother_req_f;
+      else
+        return smoother_req_d;
+    }
+
+    /// Whether the lhs of block b on level lattice g runs through stencil_column_kernel with
+    /// the operand alone in its block, so that it takes smoother steps.
+    template <typename T>
+    bool
+    smoother_fuses(int b, const GridDesc &g)
+    {
+      if (path != OperatorPath::Auto && path != OperatorPath::Split)
+        return false;
+      if (blocks[b].field_indices.size() != 1 || g.n_nodes >= stencil_min_nodes)
+        return false;
+      const SplitPlan &plan = split_plan<T>(b, true).plan;
+      const int        f    = int(*blocks[b].field_indices.begin());
+      if (!plan.eligible || plan.terms.n_terms == 0)
+        return false;
+      for (int t = 0; t < plan.terms.n_terms; ++t)
+        if (plan.terms.term[t].in_field != f ||
+            plan.terms.term[t].in_slot != prismspf::dependency_slot(prismspf::SRC))
+          return false;
+      return true;
+    }
+
+    /// Applies A (dst, src) with a smoother step attached; false if the launch did not take
+    /// the step, in which case dst holds A src.
+    template <typename T, class Vmult>
+    bool
+    smoother_step(Vmult &&A, T *dst, const T *src, Smoother kind, const SmootherArgs<T> &args)
+    {
+      auto &req = smoother_request<T>();
+      req       = {true, kind, args};
+      A(dst, src);
+      const bool taken = !req.pending;
+      req.pending      = false;
+      return taken;
+    }
+
+    /// With `fuse` set (smoother_fuses, on a level), a step is one launch that writes the new
+    /// x to the other of x and ax, whichever then holds the iterate; it starts where the
+    /// last step ends in x.
     template <typename T, class Vmult>
     void
     chebyshev(Vmult &&A, const T *inv_diag, int64_t n, unsigned int deg, double lmax,
               double lmin, T *x, const T *rhs, T *d, T *ax, bool zero_start,
-              const DiagTable<T> &tab = DiagTable<T> {})
+              const DiagTable<T> &tab = DiagTable<T> {}, bool fuse = false)
     {
       const double theta = 0.5 * (lmax + lmin);
       const double delta = 0.5 * (lmax - lmin);
       const double sigma = theta / delta;
       double       rho   = 1.0 / sigma;
+      const bool   odd   = ((zero_start ? deg - 1 : deg) & 1u) != 0;
+      T           *cur   = fuse && zero_start && odd ? ax : x;
       for (unsigned int k = 0; k < deg; ++k)
         {
           if (k == 0 && zero_start)
@@ -3204,16 +3281,15 @@ namespace ppf
               // From x = 0 the residual is b: no operator application, no clearing.
               if (tab.table)
                 hipLaunchKernelGGL(chebyshev_table_kernel<T>, class_launch(tab.grid),
-                                   dim3(256), 0, stream, x, d, rhs, (const T *)nullptr,
+                                   dim3(256), 0, stream, cur, d, rhs, (const T *)nullptr,
                                    inv_diag, tab.table, tab.ok, T(0), T(1.0 / theta), 1, 1,
                                    tab.grid);
               else
                 hipLaunchKernelGGL(chebyshev_first_zero_kernel<T>, dim3(grid_for(n, 256)),
-                                   dim3(256), 0, stream, x, d, rhs, inv_diag, T(1.0 / theta),
+                                   dim3(256), 0, stream, cur, d, rhs, inv_diag, T(1.0 / theta),
                                    n);
               continue;
             }
-          A(ax, x);
           double c1 = 0.0, c2;
           if (k == 0)
             c2 = 1.0 / theta;
@@ -3224,15 +3300,30 @@ namespace ppf
               c2                   = 2.0 * rho_new / delta;
               rho                  = rho_new;
             }
+          T *other = cur == x ? ax : x;
+          if (fuse && !(k == 0 && odd))
+            {
+              const SmootherArgs<T> args {rhs,   d,     inv_diag, tab.table,
+                                          tab.ok, T(c1), T(c2),    k == 0 ? 1 : 0};
+              if (smoother_step(A, other, cur, Smoother::Chebyshev, args))
+                {
+                  cur = other;
+                  continue;
+                }
+            }
+          else
+            A(other, cur);
           if (tab.table)
             hipLaunchKernelGGL(chebyshev_table_kernel<T>, class_launch(tab.grid), dim3(256), 0,
-                               stream, x, d, rhs, ax, inv_diag, tab.table, tab.ok, T(c1),
+                               stream, cur, d, rhs, other, inv_diag, tab.table, tab.ok, T(c1),
                                T(c2), k == 0 ? 1 : 0, 0, tab.grid);
           else
             hipLaunchKernelGGL(chebyshev_step_kernel<T>, dim3(grid_for(n, 256)), dim3(256), 0,
-                               stream, x, d, rhs, ax, inv_diag, T(c1), T(c2), k == 0 ? 1 : 0,
-                               n);
+                               stream, cur, d, rhs, other, inv_diag, T(c1), T(c2),
+                               k == 0 ? 1 : 0, n);
         }
+      if (cur != x) // a step's launch did not take the update (it ran in place)
+        copy(x, cur, n);
     }
 
     // ----------------------------------------------------------------- multigrid
@@ -3570,11 +3661,18 @@ namespace ppf
         }
       const unsigned int deg = lp.chebyshev_parameters.degree;
       const DiagTable<T> tab = level_table<T>(l, int(blocks[b].field_indices.size()));
+      const bool         fuse = smoother_fuses<T>(b, l.grid);
       chebyshev<T>(A, linv<T>(l), n, deg, l.lambda_max, l.lambda_min, lvec<T>(l, 0),
-                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), true, tab);
+                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), true, tab, fuse);
       // t = defect - A u
-      A(lvec<T>(l, 2), lvec<T>(l, 0));
-      axpby(lvec<T>(l, 2), T(1), lvec<T>(l, 1), T(-1), n);
+      SmootherArgs<T> defect;
+      defect.b = lvec<T>(l, 1);
+      const bool taken =
+        fuse && smoother_step(A, lvec<T>(l, 2), lvec<T>(l, 0), Smoother::Residual, defect);
+      if (!fuse)
+        A(lvec<T>(l, 2), lvec<T>(l, 0));
+      if (!taken)
+        axpby(lvec<T>(l, 2), T(1), lvec<T>(l, 1), T(-1), n);
       Level &c = ls.levels[li - 1];
       for (std::size_t k = 0; k < blocks[b].field_indices.size(); ++k)
         {
@@ -3590,7 +3688,7 @@ namespace ppf
                             lvec<T>(c, 0) + k * c.grid.n_nodes, c.grid, dirichlet_mask(f));
         }
       chebyshev<T>(A, linv<T>(l), n, deg, l.lambda_max, l.lambda_min, lvec<T>(l, 0),
-                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), false, tab);
+                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), false, tab, fuse);
     }
 
     /// Launch grid of a transfer kernel: a plane of e0 x e1 nodes, `groups` groups of planes.
@@ -4163,6 +4261,9 @@ namespace ppf
     DeviceBuffer<int>                              cg_done;
     DeviceBuffer<double>                           eig_slots;
     DeviceBuffer<double>                           coarse_slots;
+    /// Smoother step handed to the next lhs launch of the column kernel (smoother_step).
+    SmootherRequest<double>                        smoother_req_d;
+    SmootherRequest<float>                         smoother_req_f;
     /// Coarse-grid solve handed to the next lhs stencil launch (coarse_cg_kernel).
     CoarseCgArgs                                   coarse_req {};
     bool                                           coarse_pending = false;

@@ -167,6 +167,18 @@ namespace ppf
     return (degree == 2 && (i & 1)) ? 0 : 1;
   }
 
+  /// Node class of the inverse-diagonal tables along one axis (axis_class).
+  template <int degree>
+  PPF_HD PPF_INLINE int
+  line_class(int i, int n, int periodic)
+  {
+    if (!periodic && i == 0)
+      return 2;
+    if (!periodic && i == n - 1)
+      return 3;
+    return (degree == 2 && (i & 1)) ? 0 : 1;
+  }
+
   /// Host-side 1-D lumped mass of scale class c, in units of h.
   template <int degree>
   inline double
@@ -743,6 +755,29 @@ namespace ppf
       run(std::integral_constant<bool, false> {});
   }
 
+  /// What a smoother does with A x as stencil_column_kernel forms it, in place of storing it
+  /// for a vector kernel to read back.
+  enum class Smoother : int
+  {
+    None      = 0,
+    Chebyshev = 1, ///< r = b - A x; d = c1 d + c2 r / diag (first: c2 r / diag); out = x + d
+    Residual  = 2  ///< out = b - A x
+  };
+
+  /// Operands of a fused smoother step (one-field block vectors).  The inverse diagonal is
+  /// the class table's entry where *ok, else the array (see chebyshev_table_kernel).
+  template <typename ST>
+  struct SmootherArgs
+  {
+    const ST  *b = nullptr;
+    ST        *d = nullptr;
+    const ST  *inv_diag = nullptr;
+    const ST  *table = nullptr;
+    const int *ok = nullptr;
+    ST         c1 = ST(0), c2 = ST(0);
+    int        first = 0;
+  };
+
   /// Planes a thread of stencil_column_kernel owns.
   template <int dim>
   constexpr int stencil_column_planes = dim == 3 ? 4 : 1;
@@ -757,11 +792,15 @@ namespace ppf
   ///
   /// a.tiles_x: workgroups per plane, a.chunks_z: plane groups, a.n_blocks: their product.
   /// MASKED: some operand, input or output has Dirichlet faces.
+  ///
+  /// SM: a smoother step or residual in place of the plain result (one-field blocks whose
+  /// operand is the vector being smoothed): a Chebyshev step then moves 5 arrays instead of
+  /// 8 and takes one launch instead of two.
   template <class PDE, int dim, int degree, typename number, bool lhs, int block_id, int NF,
-            bool MASKED, typename ST = number>
+            bool MASKED, typename ST = number, Smoother SM = Smoother::None>
   __global__ void __launch_bounds__(stencil_column_threads)
   stencil_column_kernel(const PDE pde, const StencilArgs<number, ST> a, const OutTable<ST> out,
-                        const prismspf::SimulationTimer timer)
+                        const prismspf::SimulationTimer timer, const SmootherArgs<ST> sm)
   {
     constexpr int RAD = degree;
     constexpr int ZC  = stencil_column_planes<dim>;
@@ -811,6 +850,7 @@ namespace ppf
     // Every load first.
     ST column[ZC + 2 * RAD], xn[ZC][2 * RAD], yn[ZC][2 * RAD];
     ST value[ZC][NF][PPF_N_SLOTS];
+    ST sm_b[ZC], sm_d[ZC];
     if constexpr (dim == 3)
       {
 #pragma unroll
@@ -835,6 +875,10 @@ namespace ppf
 #pragma unroll
           for (int s = 0; s < PPF_N_SLOTS; ++s)
             value[k][f][s] = buffer_load<ST>(make_rsrc(a.val[f][s]), own, po);
+        if constexpr (SM != Smoother::None)
+          sm_b[k] = buffer_load<ST>(make_rsrc(sm.b), own, po);
+        if constexpr (SM == Smoother::Chebyshev)
+          sm_d[k] = buffer_load<ST>(make_rsrc(sm.d), own, po);
       }
 
     // Taps and scale factors of the column.
@@ -933,7 +977,23 @@ namespace ppf
             number acc = (fc.value_term_mask & (1u << f)) ? fc.value_term[f] : number(0);
             acc = fma(a.beta[f][0], lap, acc);
             const bool dir = MASKED && (fb & out.dirichlet_mask[f]) != 0;
-            if (!(dir && out.dirichlet_write == dirichlet_value))
+            if constexpr (SM == Smoother::Residual)
+              buffer_store(sm_b[k] - (dir ? ST(0) : ST(scale * acc)), r_dst[f], own, po,
+                           a.nt_store != 0);
+            else if constexpr (SM == Smoother::Chebyshev)
+              {
+                const ST r = sm_b[k] - (dir ? ST(0) : ST(scale * acc));
+                const unsigned int i = q + unsigned(z) * (unsigned(n0) * unsigned(n1));
+                const ST inv = sm.table && *sm.ok
+                                 ? sm.table[line_class<degree>(x, n0, p0) +
+                                            4 * line_class<degree>(y, n1, p1) +
+                                            16 * (dim == 3 ? line_class<degree>(z, n2, p2) : 1)]
+                                 : sm.inv_diag[i];
+                const ST d = sm.first ? sm.c2 * inv * r : sm.c1 * sm_d[k] + sm.c2 * inv * r;
+                buffer_store(d, make_rsrc(sm.d), own, po, false);
+                buffer_store(ST(column[dim == 3 ? k + RAD : RAD] + d), r_dst[f], own, po, false);
+              }
+            else if (!(dir && out.dirichlet_write == dirichlet_value))
               buffer_store(dir ? ST(0) : ST(scale * acc), r_dst[f], own, po, a.nt_store != 0);
           }
         if (k == 0 && a.probe_result && chk == 0 && q == 0)
