@@ -565,8 +565,8 @@ namespace ppf
     void
     axpby(T *y, T a, const T *x, T b, int64_t n)
     {
-      hipLaunchKernelGGL(axpby_kernel<T>, dim3(grid_for(n, 256)), dim3(256), 0, stream, y, a,
-                         x, b, n);
+      hipLaunchKernelGGL(axpby_kernel<T>, dim3(grid_for(n, 256 * Pack<T>::n)), dim3(256), 0,
+                         stream, y, a, x, b, n);
     }
 
     template <typename T>
@@ -1326,7 +1326,7 @@ namespace ppf
           a.beta[tm.out_field][k] += number(tm.beta);
         }
       // Two operands on a small lattice: node by node (split_operator_kernel).
-      if (a.n_ops > 1 && g.n_nodes < stencil_min_nodes && !coarse_pending &&
+      if (a.n_ops > 1 && g.n_nodes < node_kernel_limit() && !coarse_pending &&
           !(probe_req.pending && probe_req.block == b))
         return false;
       // Unused operand and value entries point at an array of the lattice size so the
@@ -1478,8 +1478,12 @@ namespace ppf
       using I4 = std::integral_constant<int, 4>;
       using I8 = std::integral_constant<int, 8>;
 
-      // Lattices below stencil_min_nodes: column by column instead of by marching tiles.
-      if (a.n_ops <= 1 && g.n_nodes < stencil_min_nodes)
+      // Lattices below stencil_min_nodes, and smoother steps: column by column instead of by
+      // marching tiles.
+      bool smoother = false;
+      if constexpr (std::is_same_v<number, ST>)
+        smoother = lhs && smoother_request<ST>().pending;
+      if (a.n_ops <= 1 && (g.n_nodes < column_kernel_limit() || smoother))
         {
           const auto go = [&](auto masked_c) {
             constexpr bool MK = decltype(masked_c)::value;
@@ -3198,9 +3202,9 @@ namespace ppf
     }
 
     static dim3
-    class_launch(const ClassGrid &g)
+    class_launch(const ClassGrid &g, int per_thread = 1)
     {
-      return dim3(grid_for(int64_t(g.n[0]) * g.n[1], 256), unsigned(g.n[2]),
+      return dim3(grid_for(int64_t(g.n[0]) * g.n[1], 256 * per_thread), unsigned(g.n[2]),
                   unsigned(g.n_fields));
     }
 
@@ -3224,6 +3228,13 @@ namespace ppf
         return smoother_req_d;
     }
 
+    /// Level lattices below this size fuse smoother steps into the operator.  Measured on the
+    /// Poisson V-cycle (Q2, per solve to 1e-8): FP64 levels up to 129^3 nodes fused take 16.2
+    /// ms, the 257^3 level fused as well 17.8 ms; FP32 levels 11.8 and 11.1 ms.
+    template <typename T>
+    static constexpr int64_t smoother_fuse_nodes =
+      std::is_same_v<T, float> ? std::numeric_limits<int64_t>::max() : int64_t(4) << 20;
+
     /// Whether the lhs of block b on level lattice g runs through stencil_column_kernel with
     /// the operand alone in its block, so that it takes smoother steps.
     template <typename T>
@@ -3232,7 +3243,8 @@ namespace ppf
     {
       if (path != OperatorPath::Auto && path != OperatorPath::Split)
         return false;
-      if (blocks[b].field_indices.size() != 1 || g.n_nodes >= stencil_min_nodes)
+      if (blocks[b].field_indices.size() != 1 || stencil_min_nodes == 0 ||
+          g.n_nodes >= std::max(column_kernel_limit(), smoother_fuse_nodes<T>))
         return false;
       const SplitPlan &plan = split_plan<T>(b, true).plan;
       const int        f    = int(*blocks[b].field_indices.begin());
@@ -3280,7 +3292,7 @@ namespace ppf
             {
               // From x = 0 the residual is b: no operator application, no clearing.
               if (tab.table)
-                hipLaunchKernelGGL(chebyshev_table_kernel<T>, class_launch(tab.grid),
+                hipLaunchKernelGGL(chebyshev_table_kernel<T>, class_launch(tab.grid, Pack<T>::n),
                                    dim3(256), 0, stream, cur, d, rhs, (const T *)nullptr,
                                    inv_diag, tab.table, tab.ok, T(0), T(1.0 / theta), 1, 1,
                                    tab.grid);
@@ -3314,8 +3326,8 @@ namespace ppf
           else
             A(other, cur);
           if (tab.table)
-            hipLaunchKernelGGL(chebyshev_table_kernel<T>, class_launch(tab.grid), dim3(256), 0,
-                               stream, cur, d, rhs, other, inv_diag, tab.table, tab.ok, T(c1),
+            hipLaunchKernelGGL(chebyshev_table_kernel<T>, class_launch(tab.grid, Pack<T>::n),
+                               dim3(256), 0, stream, cur, d, rhs, other, inv_diag, tab.table, tab.ok, T(c1),
                                T(c2), k == 0 ? 1 : 0, 0, tab.grid);
           else
             hipLaunchKernelGGL(chebyshev_step_kernel<T>, dim3(grid_for(n, 256)), dim3(256), 0,
@@ -4210,8 +4222,24 @@ namespace ppf
     /// launches whose arrays exceed stencil_nt_min_bytes).
     StorePolicy                            stencil_store_policy = StorePolicy::Auto;
     int64_t                                stencil_nt_min_bytes = int64_t(192) << 20;
-    /// Lattices with fewer nodes run split operators node by node (launch_stencil).
-    int64_t                                stencil_min_nodes    = 100000;
+    /// Lattices with fewer nodes run split operators column by column (two stencil
+    /// operands: node by node) instead of by marching tiles (launch_stencil).  Measured per
+    /// increment or application, tile / column: Cahn-Hilliard Q2 (periodic) 110k nodes 26.7 /
+    /// 17.9 us, 885k 29.3 / 25.5, 1.4M 30.6 / 32.8; precipitate Q1 885k 37.1 / 30.6, 2.1M 46.0
+    /// / 46.1; Poisson Q2 (Dirichlet) 531k FP64 13.9 / 12.9, FP32 12.3 / 10.6, 1.5M 16.3 / 20.0.
+    /// The node kernel's limit is older: BiCGStab on two operands stops on the last bits of
+    /// its sums, so those lattices keep their kernels.  Option stencil_min_nodes sets both.
+    int64_t                                stencil_min_nodes    = -1;
+    int64_t
+    column_kernel_limit() const
+    {
+      return stencil_min_nodes < 0 ? 1000000 : stencil_min_nodes;
+    }
+    int64_t
+    node_kernel_limit() const
+    {
+      return stencil_min_nodes < 0 ? 100000 : stencil_min_nodes;
+    }
     /// Start every linear solve from zero instead of the previous solution (which the
     /// reference keeps as the next initial guess, linear_solver.h:330-336).
     bool                                   zero_initial_guess    = false;
