@@ -1401,12 +1401,11 @@ namespace ppf
       if (int64_t(a.n[0]) * a.n[1] * a.n[2] * int64_t(sizeof(ST)) > (int64_t(1) << 32))
         return false;
       // Store policy: non-temporal when the distinct arrays the launch reads and writes
-      // exceed 192 MiB, i.e. cannot stay in the 256 MB Infinity Cache (the output would
-      // not be read from the caches by the next launch anyway).  Measured: the FP64 Q2
-      // Poisson apply at 257^3 nodes (271 MB) is 11 % faster with non-temporal stores,
-      // its FP32 form (136 MB) 15 % slower, and the Cahn-Hilliard increment at 129^3
-      // (51 MB per launch) 6 % slower, although each of its launches alone is faster:
-      // the next block reads the output from the caches.
+      // exceed twice the 256 MB Infinity Cache, so that none of the output would still be
+      // there for the launch that reads it.  Below that the consumer pays for it: four Poisson
+      // applications at 257^3 nodes (FP64, 271 MB each), each reading the one before, take 75
+      // us per application with temporal and 83 us with non-temporal stores (repeated on one
+      // unread output: 69 and 62 us); the Cahn-Hilliard increment at 129^3 31.3 and 33.4 us.
       {
         const void *arrays[stencil_max_ops + PPF_MAX_FIELDS * (PPF_N_SLOTS + 1)];
         int         n_arrays = 0;
@@ -1478,12 +1477,8 @@ namespace ppf
       using I4 = std::integral_constant<int, 4>;
       using I8 = std::integral_constant<int, 8>;
 
-      // Lattices below stencil_min_nodes, and smoother steps: column by column instead of by
-      // marching tiles.
-      bool smoother = false;
-      if constexpr (std::is_same_v<number, ST>)
-        smoother = lhs && smoother_request<ST>().pending;
-      if (a.n_ops <= 1 && (g.n_nodes < column_kernel_limit() || smoother))
+      // Small lattices: column by column instead of by marching tiles.
+      if (a.n_ops <= 1 && g.n_nodes < column_kernel_limit())
         {
           const auto go = [&](auto masked_c) {
             constexpr bool MK = decltype(masked_c)::value;
@@ -1581,8 +1576,11 @@ namespace ppf
           a.chunks_z = 1;
         }
       int64_t nblocks = int64_t(a.tiles_x) * a.tiles_y * a.chunks_z;
-      a.map_mode      = stencil_map;
       a.ty_per_xcd    = (a.tiles_y + 7) / 8;
+      // By size: bands on large 3-D lattices whose tile rows fill the 8 XCDs evenly.
+      const bool bands = dim == 3 && g.n_nodes >= stencil_band_nodes &&
+                         8 * 8 * a.ty_per_xcd <= 9 * a.tiles_y;
+      a.map_mode       = stencil_map >= 0 ? stencil_map : (bands ? 1 : 0);
       if (a.map_mode == 1)
         nblocks = 8 * int64_t(a.tiles_x) * a.ty_per_xcd * a.chunks_z;
       const int     wg_threads = stencil_tx * waves;
@@ -3228,23 +3226,18 @@ namespace ppf
         return smoother_req_d;
     }
 
-    /// Level lattices below this size fuse smoother steps into the operator.  Measured on the
-    /// Poisson V-cycle (Q2, per solve to 1e-8): FP64 levels up to 129^3 nodes fused take 16.2
-    /// ms, the 257^3 level fused as well 17.8 ms; FP32 levels 11.8 and 11.1 ms.
-    template <typename T>
-    static constexpr int64_t smoother_fuse_nodes =
-      std::is_same_v<T, float> ? std::numeric_limits<int64_t>::max() : int64_t(4) << 20;
-
     /// Whether the lhs of block b on level lattice g runs through stencil_column_kernel with
-    /// the operand alone in its block, so that it takes smoother steps.
+    /// the operand alone in its block, so that it takes smoother steps.  (Fused on larger
+    /// lattices as well, a Poisson solve with levels up to 257^3 Q2 nodes takes 10.7 instead
+    /// of 10.4 ms with FP32 and 17.5 instead of 15.9 ms with FP64 levels: there the tiles and
+    /// the vector kernel reach more of the bandwidth.)
     template <typename T>
     bool
     smoother_fuses(int b, const GridDesc &g)
     {
       if (path != OperatorPath::Auto && path != OperatorPath::Split)
         return false;
-      if (blocks[b].field_indices.size() != 1 || stencil_min_nodes == 0 ||
-          g.n_nodes >= std::max(column_kernel_limit(), smoother_fuse_nodes<T>))
+      if (blocks[b].field_indices.size() != 1 || g.n_nodes >= column_kernel_limit())
         return false;
       const SplitPlan &plan = split_plan<T>(b, true).plan;
       const int        f    = int(*blocks[b].field_indices.begin());
@@ -4208,8 +4201,12 @@ namespace ppf
     int                                    stencil_rows    = 0;
     int                                    stencil_waves   = 0;
     int                                    stencil_z_chunk = 0;
-    /// Workgroup -> tile order of the stencil kernel (StencilArgs::map_mode).
-    int                                    stencil_map     = 0;
+    /// Workgroup -> tile order of the stencil kernel (StencilArgs::map_mode; -1: by size).
+    /// On large lattices a band of tile rows per XCD keeps the rows and planes that tiles
+    /// share in its L2: precipitate Q1 at 7.1M nodes 126.2 -> 120.6 us per increment, Poisson
+    /// Q2 at 17M 83.6 -> 79.5 us per application; at 2.1M nodes (Cahn-Hilliard) 31.6 -> 31.9.
+    int                                    stencil_map     = -1;
+    static constexpr int64_t               stencil_band_nodes = int64_t(4) << 20;
     /// Generic path kernel: the one-pass cell-block kernel (true) or the two-pass
     /// cell/gather kernels through a global scratch array (false).
     bool                                   generic_cell_block = true;
@@ -4221,7 +4218,7 @@ namespace ppf
     /// Cache policy of the stencil kernel's output stores (Auto: non-temporal for
     /// launches whose arrays exceed stencil_nt_min_bytes).
     StorePolicy                            stencil_store_policy = StorePolicy::Auto;
-    int64_t                                stencil_nt_min_bytes = int64_t(192) << 20;
+    int64_t                                stencil_nt_min_bytes = int64_t(512) << 20;
     /// Lattices with fewer nodes run split operators column by column (two stencil
     /// operands: node by node) instead of by marching tiles (launch_stencil).  Measured per
     /// increment or application, tile / column: Cahn-Hilliard Q2 (periodic) 110k nodes 26.7 /
