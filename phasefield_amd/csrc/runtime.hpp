@@ -1493,10 +1493,20 @@ namespace ppf
             const dim3 grid {unsigned(nblocks)}, threads {stencil_column_threads};
             // A smoother waiting for A x takes the launch (see smoother_step).
             if constexpr (std::is_same_v<number, ST>)
-              if (lhs && smoother_request<ST>().pending)
+              if (lhs && smoother_request<ST>().pending &&
+                  (smoother_request<ST>().kind != Smoother::Dot || nblocks <= reduce_blocks))
                 {
                   auto &req   = smoother_request<ST>();
                   req.pending = false;
+                  req.blocks  = int(nblocks);
+                  if constexpr (std::is_same_v<ST, double>)
+                    if (req.kind == Smoother::Dot)
+                      {
+                        hipLaunchKernelGGL(
+                          (stencil_column_kernel<PDE<number>, dim, degree, number, true, id, App::n_fields, MK, ST, Smoother::Dot>),
+                          grid, threads, 0, stream, pde, a, out, timer, req.args);
+                        return true;
+                      }
                   if (req.kind == Smoother::Chebyshev)
                     hipLaunchKernelGGL(
                       (stencil_column_kernel<PDE<number>, dim, degree, number, true, id, App::n_fields, MK, ST, Smoother::Chebyshev>),
@@ -2922,16 +2932,27 @@ namespace ppf
                          d, g, ks, 1, gg, int(nb), n, 1);
       // (an enclosing halt flag keeps its meaning: no step is enqueued ahead under one)
       const unsigned int ahead = enqueue_halt ? 0 : 1;
+      const bool         fuse  = smoother_fuses<double>(b, fine);
       HaltScope          scope(*this, enqueue_halt ? enqueue_halt : done);
       unsigned int       tags[2] = {};
       const auto         enqueue = [&](unsigned int k) {
         const int cur = int((k - 1) & 1u);
-        vmult_fine(b, ls.ad.get(), d);
-        hipLaunchKernelGGL(cg_dot_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream, dad,
-                           d, ls.ad.get(), n, done);
+        // d.Ad from the operator's own launch where that is the column kernel
+        int                  sums = int(nb);
+        SmootherArgs<double> with_dot;
+        with_dot.partial = dad;
+        const auto A     = [&](double *dst, const double *src) { vmult_fine(b, dst, src); };
+        if (fuse && smoother_step(A, ls.ad.get(), (const double *) d, Smoother::Dot, with_dot))
+          sums = smoother_request<double>().blocks;
+        else
+          {
+            if (!fuse)
+              A(ls.ad.get(), d);
+            hipLaunchKernelGGL(cg_dot_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream,
+                               dad, d, ls.ad.get(), n, done);
+          }
         hipLaunchKernelGGL(cg_step_kernel<double>, dim3(nb), dim3(reduce_threads), 0, stream, gg,
-                           x, g, (double *) nullptr, d, ls.ad.get(), ks, cur, dad, int(nb), n,
-                           done);
+                           x, g, (double *) nullptr, d, ls.ad.get(), ks, cur, dad, sums, n, done);
         tags[k & 1u] = next_host_tag();
         hipLaunchKernelGGL(cg_turn_kernel, dim3(nb), dim3(reduce_threads), 0, stream, d, g, ks,
                            cur, gg, int(nb), n, tol, done, host_scalar(tags[k & 1u]),
@@ -3214,6 +3235,7 @@ namespace ppf
       bool            pending = false;
       Smoother        kind    = Smoother::None;
       SmootherArgs<T> args {};
+      int             blocks = 0; ///< workgroups of the launch that took it
     };
 
     template <typename T>
@@ -3257,7 +3279,7 @@ namespace ppf
     smoother_step(Vmult &&A, T *dst, const T *src, Smoother kind, const SmootherArgs<T> &args)
     {
       auto &req = smoother_request<T>();
-      req       = {true, kind, args};
+      req       = {true, kind, args, 0};
       A(dst, src);
       const bool taken = !req.pending;
       req.pending      = false;

@@ -761,7 +761,8 @@ namespace ppf
   {
     None      = 0,
     Chebyshev = 1, ///< r = b - A x; d = c1 d + c2 r / diag (first: c2 r / diag); out = x + d
-    Residual  = 2  ///< out = b - A x
+    Residual  = 2, ///< out = b - A x
+    Dot       = 3  ///< out = A x, and per-workgroup partial sums of x . A x (CG)
   };
 
   /// Operands of a fused smoother step (one-field block vectors).  The inverse diagonal is
@@ -776,6 +777,7 @@ namespace ppf
     const int *ok = nullptr;
     ST         c1 = ST(0), c2 = ST(0);
     int        first = 0;
+    double    *partial = nullptr;
   };
 
   /// Planes a thread of stencil_column_kernel owns.
@@ -814,10 +816,13 @@ namespace ppf
     const int b   = blockIdx.x;
     const int lb  = b < 8 * q8 ? (b % 8) * q8 + b / 8 : b;
     const int chk = lb / a.tiles_x;
-    const unsigned int q =
-      unsigned(lb - chk * a.tiles_x) * stencil_column_threads + threadIdx.x;
-    if (q >= unsigned(n0) * unsigned(n1))
+    unsigned int q = unsigned(lb - chk * a.tiles_x) * stencil_column_threads + threadIdx.x;
+    const bool   inside = q < unsigned(n0) * unsigned(n1);
+    if (SM != Smoother::Dot && !inside)
       return;
+    if (SM == Smoother::Dot && !inside)
+      q = 0; // computes node 0's column, stores nothing: the workgroup sums together
+    double dot = 0.0;
     const int          y  = int(q / unsigned(n0));
     const int          x  = int(q - unsigned(y) * unsigned(n0));
     const int          z0 = chk * ZC;
@@ -993,11 +998,26 @@ namespace ppf
                 buffer_store(d, make_rsrc(sm.d), own, po, false);
                 buffer_store(ST(column[dim == 3 ? k + RAD : RAD] + d), r_dst[f], own, po, false);
               }
+            else if constexpr (SM == Smoother::Dot)
+              {
+                const ST ax = dir ? ST(0) : ST(scale * acc);
+                if (inside)
+                  {
+                    buffer_store(ax, r_dst[f], own, po, a.nt_store != 0);
+                    dot += double(column[dim == 3 ? k + RAD : RAD]) * double(ax);
+                  }
+              }
             else if (!(dir && out.dirichlet_write == dirichlet_value))
               buffer_store(dir ? ST(0) : ST(scale * acc), r_dst[f], own, po, a.nt_store != 0);
           }
         if (k == 0 && a.probe_result && chk == 0 && q == 0)
           stencil_probe(a);
+      }
+    if constexpr (SM == Smoother::Dot)
+      {
+        dot = block_sum(dot);
+        if (threadIdx.x == 0)
+          sm.partial[blockIdx.x] = dot;
       }
   }
 
