@@ -103,7 +103,7 @@ int ppf_field_name(ppf_ctx *ctx, int field, char *buf, int len);
  * "stencil_z_chunk" = <planes> (0: automatic) tune the tiled kernel's workgroup
  * shape; "stencil_min_nodes" = <n>: lattices with fewer
  * nodes run split operators column by column instead of by tiles, those with two stencil
- * operands node by node (defaults 1000000 and 100000; 0: tiles at any size); "stencil_store_policy" = auto|temporal|nontemporal sets the cache policy of
+ * operands node by node (defaults 1000000, in 2-D 500000, and 100000; 0: tiles at any size); "stencil_store_policy" = auto|temporal|nontemporal sets the cache policy of
  * its output stores (auto: non-temporal when the launch's arrays exceed 512 MiB);
  * "generic_kernel" = cell_block|two_pass selects the generic path's kernels (cell_block:
  * one launch, cell blocks staged in shared memory, no device scratch; two_pass: a cell

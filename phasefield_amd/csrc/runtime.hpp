@@ -945,23 +945,24 @@ namespace ppf
                 oref.dst[bf[k]] = ref + int64_t(k) * n;
               launch(false, oref);
               launch(true, out);
-              double worst = 0.0, scale = 0.0;
+              // Partial maxima of all fields, one copy and one wait (a wait per field made the
+              // first use of a small coupled plan 50 us longer).
+              const int           parts = reduce_blocks / int(bf.size());
+              double              worst = 0.0, scale = 0.0;
+              std::vector<double> part(2 * parts * bf.size());
               for (std::size_t k = 0; k < bf.size(); ++k)
-                {
-                  hipLaunchKernelGGL(max_diff_partial_kernel<number>, dim3(reduce_blocks),
-                                     dim3(reduce_threads), 0, stream, reduce_buf.get(),
-                                     dst[k], oref.dst[bf[k]], n);
-                  std::vector<double> part(2 * reduce_blocks);
-                  PPF_HIP_CHECK(hipMemcpyAsync(part.data(), reduce_buf.get(),
-                                               sizeof(double) * part.size(),
-                                               hipMemcpyDeviceToHost, stream));
-                  sync();
-                  for (int i = 0; i < reduce_blocks; ++i)
-                    {
-                      worst = std::max(worst, part[i]);
-                      scale = std::max(scale, part[reduce_blocks + i]);
-                    }
-                }
+                hipLaunchKernelGGL(max_diff_partial_kernel<number>, dim3(parts),
+                                   dim3(reduce_threads), 0, stream,
+                                   reduce_buf.get() + 2 * parts * k, dst[k], oref.dst[bf[k]], n);
+              PPF_HIP_CHECK(hipMemcpyAsync(part.data(), reduce_buf.get(),
+                                           sizeof(double) * part.size(), hipMemcpyDeviceToHost,
+                                           stream));
+              sync();
+              for (std::size_t i = 0; i < part.size(); ++i)
+                if ((i / parts) % 2 == 0)
+                  worst = std::max(worst, part[i]);
+                else
+                  scale = std::max(scale, part[i]);
               int halted_now = 0;
               if (out.halt)
                 PPF_HIP_CHECK(hipMemcpy(&halted_now, out.halt, sizeof(int),
@@ -4246,13 +4247,14 @@ namespace ppf
     /// increment or application, tile / column: Cahn-Hilliard Q2 (periodic) 110k nodes 26.7 /
     /// 17.9 us, 885k 29.3 / 25.5, 1.4M 30.6 / 32.8; precipitate Q1 885k 37.1 / 30.6, 2.1M 46.0
     /// / 46.1; Poisson Q2 (Dirichlet) 531k FP64 13.9 / 12.9, FP32 12.3 / 10.6, 1.5M 16.3 / 20.0.
+    /// In 2-D (Allen-Cahn Q1) 250k nodes 7.0 / 6.9, 490k 7.19 / 7.17, 790k 8.55 / 8.93.
     /// The node kernel's limit is older: BiCGStab on two operands stops on the last bits of
     /// its sums, so those lattices keep their kernels.  Option stencil_min_nodes sets both.
     int64_t                                stencil_min_nodes    = -1;
     int64_t
     column_kernel_limit() const
     {
-      return stencil_min_nodes < 0 ? 1000000 : stencil_min_nodes;
+      return stencil_min_nodes < 0 ? (dim == 3 ? 1000000 : 500000) : stencil_min_nodes;
     }
     int64_t
     node_kernel_limit() const
