@@ -13,6 +13,7 @@
 #include "coupled_kernels.hpp"
 #include "device.hpp"
 #include "grid.hpp"
+#include "host_scalars.hpp"
 #include "operator_kernels.hpp"
 #include "operator_plan.hpp"
 #include "pair_kernels.hpp"
@@ -608,19 +609,17 @@ namespace ppf
       return wait_host_scalar(tag).first;
     }
 
-    /// Tag of the next scalar sent to the host, and the ring entry it goes to: at most two
-    /// are under way at a time, so an entry is read before its next use.
+    /// Tag of the next scalar sent to the host, and the entry it goes to.
     unsigned int
     next_host_tag()
     {
-      host_tag = (host_tag + 1) & 0x7fffffffu;
-      return host_tag;
+      return host_ring.issue(host_scalars.get(HostScalarRing::size));
     }
 
     HostScalar *
     host_scalar(unsigned int tag)
     {
-      return host_scalars.get(host_scalar_ring) + tag % host_scalar_ring;
+      return HostScalarRing::entry(host_scalars.get(HostScalarRing::size), tag);
     }
 
     /// Waits for the scalar with this tag by polling its pinned entry (a copy and a stream
@@ -630,11 +629,9 @@ namespace ppf
     {
       ++sync_count_;
       const HostScalar *entry = host_scalar(tag);
-      const auto        ready = [&](unsigned int w) { return (w >> 1) == tag; };
-      const auto        word  = [&] {
-        return *reinterpret_cast<const volatile unsigned int *>(&entry->word);
-      };
-      unsigned int w = word();
+      const auto        ready = [&](unsigned int w) { return HostScalarRing::ready(w, tag); };
+      const auto        word  = [&] { return HostScalarRing::word(entry); };
+      unsigned int      w     = word();
       for (unsigned long spin = 1; !ready(w); ++spin, w = word())
         if (spin % 4096 == 0)
           {
@@ -4304,9 +4301,8 @@ namespace ppf
     DeviceBuffer<float>                            zeros_f;
     DeviceBuffer<double>                           reduce_buf;
     /// Scalars the host polls for (finish_reduction, cg).
-    static constexpr int                           host_scalar_ring = 4;
     PinnedBuffer<HostScalar>                       host_scalars;
-    unsigned int                                   host_tag = 0;
+    HostScalarRing                                 host_ring;
     DeviceBuffer<int>                              cg_done;
     DeviceBuffer<double>                           eig_slots;
     DeviceBuffer<double>                           coarse_slots;

@@ -7,6 +7,7 @@
 #pragma once
 
 #include "grid.hpp"
+#include "host_scalars.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -368,13 +369,7 @@ namespace ppf
     return block_total(s);
   }
 
-  /// A scalar for the polling host: value, then (tag << 1) | flag once it is visible.
-  struct HostScalar
-  {
-    double       value;
-    unsigned int word;
-  };
-
+  /// Sends a scalar to the polling host.
   __device__ PPF_INLINE void
   tell_host(HostScalar *to, double value, unsigned int tag, bool flag)
   {

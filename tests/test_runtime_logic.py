@@ -1,0 +1,26 @@
+"""Host logic of the runtime on the CPU: small headers of phasefield_amd/csrc compiled into
+native programs (no GPU calls)."""
+
+from __future__ import annotations
+
+import subprocess
+from pathlib import Path
+
+ROOT = Path(__file__).resolve().parent.parent
+
+
+def native(tmp_path, name, compiler=("g++",)):
+    """Compiles tests/native/<name>, runs it and returns its "key: value" lines."""
+    exe = tmp_path / Path(name).stem
+    subprocess.run([*compiler, "-std=c++20", "-O1", f"-I{ROOT / 'phasefield_amd' / 'include'}",
+                    f"-I{ROOT / 'phasefield_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "native" / name), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout
+    return dict(line.split(": ", 1) for line in out.splitlines())
+
+
+def test_host_scalars_ignore_what_the_memory_held(tmp_path):
+    out = native(tmp_path, "host_scalars.cc")
+    # no entry counts as sent before its scalar is, also not one with the awaited tag
+    assert out["first"] == "1" and out["stale"] == "0" and out["missed"] == "0"
+    assert out["last"] == str(2 ** 31 - 1) and out["wrapped"] == "1" and out["empty"] == "0"
