@@ -324,13 +324,14 @@ namespace ppf
 
   // ---------------------------------------------------------------- CG iteration
   //
-  // A step is: operator application, d.Ad partial sums, cg_step_kernel, and either
-  // cg_turn_kernel (no preconditioner: h = g) or cg_residual_kernel, preconditioner, g.h
-  // partial sums and cg_direction_kernel.  No kernel only finishes a sum: every workgroup
-  // of the kernel that needs a dot product adds the few hundred partial sums itself, in one
-  // fixed order (8 kB from L2; a reduction kernel of its own costs a launch, about 5 us of
-  // a 45 us step at 140k nodes).  The residual norm goes to pinned host memory, which the
-  // host polls, so that no copy or stream synchronization ends a step.
+  // A step is: operator application, d.Ad partial sums (by the operator's own launch where
+  // that takes them), cg_step_kernel, and either cg_turn_kernel (no preconditioner: h = g) or
+  // reduce_to_host_kernel, preconditioner, g.h partial sums and cg_direction_kernel.  Sums
+  // that only the device needs have no kernel that finishes them: every workgroup of the
+  // kernel that uses a dot product adds the few hundred partial sums itself, in one fixed
+  // order (8 kB from L2; a reduction kernel of its own costs a launch, about 5 us of a 45 us
+  // step at 140k nodes).  The residual norm goes to pinned host memory, which the host polls,
+  // so that no copy or stream synchronization ends a step.
 
   /// Workgroups (and partial sums) of the kernels below for vectors of length n: one element
   /// per thread until every compute unit has a workgroup (with four, 66k elements used 65 of
@@ -433,6 +434,16 @@ namespace ppf
       partial_gg[blockIdx.x] = acc;
   }
 
+  /// *done holds the tag of the scalar with which a CG iteration ended, 0 before.  Whether the
+  /// cg_turn_kernel launch with scalar `tag` follows that end: not if it is the launch that
+  /// sets *done, whose waves read the word while workgroup 0 stores it.  Either value they find
+  /// then takes all of them into the sums below, with barriers, and out by their result.
+  PPF_HD PPF_INLINE bool
+  cg_ended_before(int done, unsigned int tag)
+  {
+    return done != 0 && (unsigned int) done != tag;
+  }
+
   /// Unpreconditioned end of a step: gg = g.g (also the next g.h); if |g| <= tol (or it is
   /// not a number) *done is set and d stays, else d = -g + (gg / s[cur]) d and s[1 - cur] =
   /// gg.  Tells the host gg and whether the iteration is done.
@@ -441,17 +452,15 @@ namespace ppf
                  int cur, const double *__restrict__ partial_gg, int count, int64_t n,
                  double tol, int *done, HostScalar *to, unsigned int tag)
   {
-    if (*done)
+    if (cg_ended_before(__hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), tag))
       return;
     const double gg  = sum_partials(partial_gg, count);
     const bool   end = !(std::sqrt(gg) > tol);
     if (blockIdx.x == 0 && threadIdx.x == 0)
       {
         tell_host(to, gg, tag, end);
-        // A block of this launch that starts after this store leaves at once, as it would
-        // have by `end`.
         if (end)
-          *done = 1;
+          __hip_atomic_store(done, int(tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     if (end)
       return;

@@ -6,6 +6,10 @@ from __future__ import annotations
 import subprocess
 from pathlib import Path
 
+import pytest
+
+from phasefield_amd.build import HIP_FLAGS, HIPCC
+
 ROOT = Path(__file__).resolve().parent.parent
 
 
@@ -24,3 +28,17 @@ def test_host_scalars_ignore_what_the_memory_held(tmp_path):
     # no entry counts as sent before its scalar is, also not one with the awaited tag
     assert out["first"] == "1" and out["stale"] == "0" and out["missed"] == "0"
     assert out["last"] == str(2 ** 31 - 1) and out["wrapped"] == "1" and out["empty"] == "0"
+
+
+@pytest.fixture(scope="module")
+def logic(tmp_path_factory):
+    """Host evaluations of functions that the kernels and their launches share."""
+    return native(tmp_path_factory.mktemp("logic"), "runtime_logic.hip",
+                  (HIPCC, *(f for f in HIP_FLAGS if f != "-shared")))
+
+
+def test_cg_turn_is_uniform_while_it_ends(logic):
+    # A launch whose waves find 0 or the launch's own tag, by when they look, must not part:
+    # both stay for the barriers of its sums.  Only later launches leave at once.
+    assert logic["turn_open"] == "00" and logic["turn_racing"] == "0"
+    assert logic["turn_after"] == "1" and logic["turn_last_tag"] == "10"
