@@ -17,6 +17,7 @@
 #include "operator_kernels.hpp"
 #include "operator_plan.hpp"
 #include "pair_kernels.hpp"
+#include "smoother_request.hpp"
 #include "stencil_kernels.hpp"
 #include "vector_kernels.hpp"
 #include "vtu_writer.hpp"
@@ -1491,12 +1492,12 @@ namespace ppf
             const dim3 grid {unsigned(nblocks)}, threads {stencil_column_threads};
             // A smoother waiting for A x takes the launch (see smoother_step).
             if constexpr (std::is_same_v<number, ST>)
-              if (lhs && smoother_request<ST>().pending &&
-                  (smoother_request<ST>().kind != Smoother::Dot || nblocks <= reduce_blocks))
+              if (auto &req = smoother_request<ST>();
+                  lhs && a.n_ops == 1 &&
+                  req.waits_for(b, out.dst[*blocks[b].field_indices.begin()], a.op[0]) &&
+                  (req.kind != Smoother::Dot || nblocks <= reduce_blocks))
                 {
-                  auto &req   = smoother_request<ST>();
-                  req.pending = false;
-                  req.blocks  = int(nblocks);
+                  req.take(int(nblocks));
                   if constexpr (std::is_same_v<ST, double>)
                     if (req.kind == Smoother::Dot)
                       {
@@ -2940,7 +2941,7 @@ namespace ppf
         SmootherArgs<double> with_dot;
         with_dot.partial = dad;
         const auto A     = [&](double *dst, const double *src) { vmult_fine(b, dst, src); };
-        if (fuse && smoother_step(A, ls.ad.get(), (const double *) d, Smoother::Dot, with_dot))
+        if (fuse && smoother_step(b, A, ls.ad.get(), (const double *) d, Smoother::Dot, with_dot))
           sums = smoother_request<double>().blocks;
         else
           {
@@ -3225,17 +3226,7 @@ namespace ppf
                   unsigned(g.n_fields));
     }
 
-    /// A smoother step (Chebyshev update or residual) waiting for the operator application
-    /// that forms its A x.
-    template <typename T>
-    struct SmootherRequest
-    {
-      bool            pending = false;
-      Smoother        kind    = Smoother::None;
-      SmootherArgs<T> args {};
-      int             blocks = 0; ///< workgroups of the launch that took it
-    };
-
+    /// The smoother step waiting for its operator application, if any.
     template <typename T>
     SmootherRequest<T> &
     smoother_request()
@@ -3270,29 +3261,34 @@ namespace ppf
       return true;
     }
 
-    /// Applies A (dst, src) with a smoother step attached; false if the launch did not take
-    /// the step, in which case dst holds A src.
+    /// Applies A (dst, src), the lhs of block b, with a smoother step attached; false if the
+    /// launch did not take the step, in which case dst holds A src.
     template <typename T, class Vmult>
     bool
-    smoother_step(Vmult &&A, T *dst, const T *src, Smoother kind, const SmootherArgs<T> &args)
+    smoother_step(int b, Vmult &&A, T *dst, const T *src, Smoother kind,
+                  const SmootherArgs<T> &args)
     {
-      auto &req = smoother_request<T>();
-      req       = {true, kind, args, 0};
+      SmootherRequest<T> request;
+      request.block = b;
+      request.dst   = dst;
+      request.src   = src;
+      request.kind  = kind;
+      request.args  = args;
+      SmootherScope<T> scope(smoother_request<T>(), request);
       A(dst, src);
-      const bool taken = !req.pending;
-      req.pending      = false;
-      return taken;
+      return scope.slot.taken;
     }
 
-    /// With `fuse` set (smoother_fuses, on a level), a step is one launch that writes the new
-    /// x to the other of x and ax, whichever then holds the iterate; it starts where the
-    /// last step ends in x.
+    /// With `fuse_block` set (A is the lhs of that block, smoother_fuses), a step is one launch
+    /// that writes the new x to the other of x and ax, whichever then holds the iterate; it
+    /// starts where the last step ends in x.
     template <typename T, class Vmult>
     void
     chebyshev(Vmult &&A, const T *inv_diag, int64_t n, unsigned int deg, double lmax,
               double lmin, T *x, const T *rhs, T *d, T *ax, bool zero_start,
-              const DiagTable<T> &tab = DiagTable<T> {}, bool fuse = false)
+              const DiagTable<T> &tab = DiagTable<T> {}, int fuse_block = -1)
     {
+      const bool   fuse  = fuse_block >= 0;
       const double theta = 0.5 * (lmax + lmin);
       const double delta = 0.5 * (lmax - lmin);
       const double sigma = theta / delta;
@@ -3330,7 +3326,7 @@ namespace ppf
             {
               const SmootherArgs<T> args {rhs,   d,     inv_diag, tab.table,
                                           tab.ok, T(c1), T(c2),    k == 0 ? 1 : 0};
-              if (smoother_step(A, other, cur, Smoother::Chebyshev, args))
+              if (smoother_step(fuse_block, A, other, cur, Smoother::Chebyshev, args))
                 {
                   cur = other;
                   continue;
@@ -3686,14 +3682,15 @@ namespace ppf
         }
       const unsigned int deg = lp.chebyshev_parameters.degree;
       const DiagTable<T> tab = level_table<T>(l, int(blocks[b].field_indices.size()));
-      const bool         fuse = smoother_fuses<T>(b, l.grid);
+      const bool         fuse       = smoother_fuses<T>(b, l.grid);
+      const int          fuse_block = fuse ? b : -1;
       chebyshev<T>(A, linv<T>(l), n, deg, l.lambda_max, l.lambda_min, lvec<T>(l, 0),
-                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), true, tab, fuse);
+                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), true, tab, fuse_block);
       // t = defect - A u
       SmootherArgs<T> defect;
       defect.b = lvec<T>(l, 1);
       const bool taken =
-        fuse && smoother_step(A, lvec<T>(l, 2), lvec<T>(l, 0), Smoother::Residual, defect);
+        fuse && smoother_step<T>(b, A, lvec<T>(l, 2), lvec<T>(l, 0), Smoother::Residual, defect);
       if (!fuse)
         A(lvec<T>(l, 2), lvec<T>(l, 0));
       if (!taken)
@@ -3713,7 +3710,7 @@ namespace ppf
                             lvec<T>(c, 0) + k * c.grid.n_nodes, c.grid, dirichlet_mask(f));
         }
       chebyshev<T>(A, linv<T>(l), n, deg, l.lambda_max, l.lambda_min, lvec<T>(l, 0),
-                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), false, tab, fuse);
+                   lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), false, tab, fuse_block);
     }
 
     /// Launch grid of a transfer kernel: a plane of e0 x e1 nodes, `groups` groups of planes.

@@ -42,6 +42,7 @@
 
 #include "operator_kernels.hpp"
 #include "vector_kernels.hpp"
+#include "smoother_request.hpp"
 
 #include <type_traits>
 #include <utility>
@@ -754,31 +755,6 @@ namespace ppf
     else
       run(std::integral_constant<bool, false> {});
   }
-
-  /// What a smoother does with A x as stencil_column_kernel forms it, in place of storing it
-  /// for a vector kernel to read back.
-  enum class Smoother : int
-  {
-    None      = 0,
-    Chebyshev = 1, ///< r = b - A x; d = c1 d + c2 r / diag (first: c2 r / diag); out = x + d
-    Residual  = 2, ///< out = b - A x
-    Dot       = 3  ///< out = A x, and per-workgroup partial sums of x . A x (CG)
-  };
-
-  /// Operands of a fused smoother step (one-field block vectors).  The inverse diagonal is
-  /// the class table's entry where *ok, else the array (see chebyshev_table_kernel).
-  template <typename ST>
-  struct SmootherArgs
-  {
-    const ST  *b = nullptr;
-    ST        *d = nullptr;
-    const ST  *inv_diag = nullptr;
-    const ST  *table = nullptr;
-    const int *ok = nullptr;
-    ST         c1 = ST(0), c2 = ST(0);
-    int        first = 0;
-    double    *partial = nullptr;
-  };
 
   /// Planes a thread of stencil_column_kernel owns.
   template <int dim>

@@ -42,3 +42,12 @@ def test_cg_turn_is_uniform_while_it_ends(logic):
     # both stay for the barriers of its sums.  Only later launches leave at once.
     assert logic["turn_open"] == "00" and logic["turn_racing"] == "0"
     assert logic["turn_after"] == "1" and logic["turn_last_tag"] == "10"
+
+
+def test_smoother_step_is_for_its_application_only(tmp_path):
+    out = native(tmp_path, "smoother_request.cc")
+    assert out["own"] == "10" and out["taken"] == "017"
+    for other in ("before", "other_block", "other_dst", "other_src"):
+        assert out[other] == "0", other
+    # nothing is left for the next launch where the application threw or did not take it
+    assert out["after_throw"] == "00" and out["not_taken"] == "00"
