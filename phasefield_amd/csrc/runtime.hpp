@@ -938,6 +938,9 @@ namespace ppf
             }
           if (ref)
             {
+              // A x itself is compared, and the partial sums below are reduce_buf's: a smoother
+              // step waiting for this application is left to the vector kernels.
+              smoother_request<number>().withdraw();
               OutTable<number> oref = out;
               for (std::size_t k = 0; k < bf.size(); ++k)
                 oref.dst[bf[k]] = ref + int64_t(k) * n;

@@ -51,6 +51,13 @@ namespace ppf
       return pending && block == b && dst == to && src == from;
     }
 
+    /// No launch is to carry the step out: the application gives A x.
+    void
+    withdraw()
+    {
+      pending = false;
+    }
+
     /// A launch of n workgroups carries the step out.
     void
     take(int n)

@@ -25,6 +25,12 @@ main()
     slot.take(7);
     std::cout << "taken: " << slot.waits_for(2, y, x) << slot.taken << slot.blocks << "\n";
   }
+  {
+    // an application that compares two paths on A x
+    SmootherScope<double> scope(slot, step);
+    slot.withdraw();
+    std::cout << "withdrawn: " << slot.waits_for(2, y, x) << slot.taken << "\n";
+  }
   // an application that throws, one that no launch took, and a second one after each
   try
     {

@@ -49,5 +49,7 @@ def test_smoother_step_is_for_its_application_only(tmp_path):
     assert out["own"] == "10" and out["taken"] == "017"
     for other in ("before", "other_block", "other_dst", "other_src"):
         assert out[other] == "0", other
+    # an application that compares A x takes none, and says so to the caller
+    assert out["withdrawn"] == "00"
     # nothing is left for the next launch where the application threw or did not take it
     assert out["after_throw"] == "00" and out["not_taken"] == "00"
