@@ -3716,16 +3716,6 @@ namespace ppf
                    lvec<T>(l, 1), lvec<T>(l, 3), lvec<T>(l, 4), false, tab, fuse_block);
     }
 
-    /// Launch grid of a transfer kernel: a plane of e0 x e1 nodes, `groups` groups of planes.
-    static dim3
-    transfer_grid(int e0, int e1, int groups)
-    {
-      const int64_t plane = int64_t(e0) * e1;
-      if (plane >= (int64_t(1) << 31) || groups > 65535)
-        throw Error(status_unsupported, "transfer: lattice too large for one launch");
-      return dim3(grid_for(plane, transfer_threads), unsigned(groups));
-    }
-
     /// fine += P coarse (fine Dirichlet nodes untouched).
     template <typename T>
     void
@@ -3735,7 +3725,7 @@ namespace ppf
       const int zc     = 2 * degree;
       const int layers = dim == 3 ? (gf.nodes[2] + zc - 1) / zc : 1;
       hipLaunchKernelGGL((prolongate_add_kernel<dim, degree, T>),
-                         transfer_grid(gf.nodes[0], gf.nodes[1], layers), dim3(transfer_threads),
+                         transfer_grid(gf, gc, gf, layers), dim3(transfer_threads),
                          0, stream, fine_v, coarse_v, gc, gf, mask);
     }
 
@@ -3748,7 +3738,7 @@ namespace ppf
       constexpr int zc     = restrict_planes<dim>;
       const int     groups = dim == 3 ? (gc.nodes[2] + zc - 1) / zc : 1;
       hipLaunchKernelGGL((restrict_kernel<dim, degree, T>),
-                         transfer_grid(gc.nodes[0], gc.nodes[1], groups), dim3(transfer_threads),
+                         transfer_grid(gc, gc, gf, groups), dim3(transfer_threads),
                          0, stream, coarse_v, fine_v, gc, gf, mask);
     }
 

@@ -6,6 +6,7 @@
 // rank count too).
 #pragma once
 
+#include "device.hpp"
 #include "grid.hpp"
 #include "host_scalars.hpp"
 
@@ -947,6 +948,19 @@ namespace ppf
   template <int dim>
   constexpr int restrict_planes = dim == 3 ? 4 : 1;
   constexpr int transfer_threads = 256;
+
+  /// Launch grid of a transfer between the lattices gc and gf: the x-y plane of `out` (either),
+  /// `groups` groups of its planes.  Both kernels index a plane of both lattices with 32 bits;
+  /// the fine one is the larger, also where the launch runs over the coarse one.
+  inline dim3
+  transfer_grid(const GridDesc &out, const GridDesc &gc, const GridDesc &gf, int groups)
+  {
+    for (const GridDesc *g : {&gc, &gf})
+      if (int64_t(g->nodes[0]) * g->nodes[1] >= (int64_t(1) << 31) || g->nodes[2] > 65535)
+        throw Error(status_unsupported, "transfer: lattice too large for one launch");
+    return dim3(grid_for(int64_t(out.nodes[0]) * out.nodes[1], transfer_threads),
+                unsigned(groups));
+  }
 
   /// coarse = P^T fine (transposed 1-D weights per axis), zero at the coarse Dirichlet nodes.
   /// Grid: x over the coarse plane, y over groups of restrict_planes planes.

@@ -53,3 +53,9 @@ def test_smoother_step_is_for_its_application_only(tmp_path):
     assert out["withdrawn"] == "00"
     # nothing is left for the next launch where the application threw or did not take it
     assert out["after_throw"] == "00" and out["not_taken"] == "00"
+
+
+def test_transfer_launches_check_both_planes(logic):
+    # The restriction runs over the coarse plane and reads the fine one with 32-bit indices.
+    assert logic["transfer_fits"] == "00"
+    assert logic["transfer_fine_plane"] == "1111" and logic["transfer_planes"] == "11"
