@@ -897,11 +897,12 @@ namespace ppf
   /// lattice (flattened, so that no lane idles at a ragged width) and sums the x and y taps
   /// of a plane in registers before the z taps, which needs no intermediate lattices.  (A
   /// pass per axis moved the fine vector three times: at 257^3 FP32 the restriction took
-  /// about 100 us and the prolongation 130 us.)  Every output takes a fixed number of taps;
-  /// taps that do not occur or lie outside a non-periodic lattice have weight zero.
+  /// about 100 us and the prolongation 130 us.)  Every output takes a fixed number of taps.
+  /// One that does not occur or lies outside a non-periodic lattice has weight zero and the
+  /// position of one that counts: a NaN or an infinity reaches only the outputs that take it.
 
   /// Taps of the restriction along one axis at coarse coordinate J: fine positions and
-  /// weights, in the order 2J, 2J - 1, 2J + 1, 2J - 3, 2J + 3.
+  /// weights, in the order 2J (always there), 2J - 1, 2J + 1, 2J - 3, 2J + 3.
   template <int degree>
   constexpr int restrict_taps = degree == 1 ? 3 : 5;
 
@@ -924,7 +925,7 @@ namespace ppf
   }
 
   template <int degree, typename T>
-  __device__ PPF_INLINE void
+  PPF_HD PPF_INLINE void
   restrict_axis(int J, int n, int periodic, int (&pos)[restrict_taps<degree>],
                 T (&w)[restrict_taps<degree>])
   {
@@ -938,8 +939,9 @@ namespace ppf
           i = i < 0 ? i + n : (i >= n ? i - n : i);
         else
           ok = i >= 0 && i < n;
-        pos[k] = ok ? i : 0;
-        w[k]   = ok ? T(restrict_weight<degree>(k, even)) : T(0);
+        const double weight = ok ? restrict_weight<degree>(k, even) : 0.0;
+        pos[k]              = weight != 0.0 ? i : 2 * J;
+        w[k]                = T(weight);
       }
   }
 
@@ -1050,16 +1052,13 @@ namespace ppf
   /// Taps of the prolongation along one axis at fine coordinate I: coarse positions
   /// b .. b + degree of its coarse cell and their weights (an even I is a coarse node).
   template <int degree, typename T>
-  __device__ PPF_INLINE void
+  PPF_HD PPF_INLINE void
   prolong_axis(int I, int n, int periodic, int (&pos)[degree + 1], T (&w)[degree + 1])
   {
     const int b = degree * (I / (2 * degree)), r = I % (2 * degree);
 #pragma unroll
     for (int k = 0; k <= degree; ++k)
       {
-        int i  = b + k;
-        i      = i >= n ? (periodic ? i - n : n - 1) : i; // beyond the lattice: weight zero
-        pos[k] = i;
         double v;
         if (degree == 1)
           v = r == 0 ? (k == 0 ? 1.0 : 0.0) : 0.5;
@@ -1067,7 +1066,10 @@ namespace ppf
           v = k == r / 2 ? 1.0 : 0.0;
         else
           v = k == 1 ? 3.0 / 4.0 : ((k == 0) == (r == 1) ? 3.0 / 8.0 : -1.0 / 8.0);
-        w[k] = T(v);
+        // weight zero only where I is the coarse node b + r / 2
+        const int i = b + (v != 0.0 ? k : r / 2);
+        pos[k]      = i >= n && periodic ? i - n : i;
+        w[k]        = T(v);
       }
   }
 

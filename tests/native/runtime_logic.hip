@@ -33,6 +33,50 @@ namespace
         }
     return r;
   }
+
+  /// Taps of weight zero whose position no tap of the same output has with another weight, and
+  /// positions outside the lattice that is read.
+  template <int taps>
+  void
+  count(const int (&pos)[taps], const double (&w)[taps], int n, int &stray, int &outside)
+  {
+    for (int k = 0; k < taps; ++k)
+      {
+        bool counts = false;
+        for (int m = 0; m < taps; ++m)
+          counts = counts || (pos[m] == pos[k] && w[m] != 0.0);
+        stray += !counts;
+        outside += pos[k] < 0 || pos[k] >= n;
+      }
+  }
+
+  template <int degree>
+  void
+  transfer_taps()
+  {
+    int stray[2] = {}, outside[2] = {};
+    for (int periodic = 0; periodic < 2; ++periodic)
+      for (int cells = 1; cells <= 5; ++cells) // of the coarse lattice
+        {
+          const int nc = degree * cells + !periodic, nf = 2 * degree * cells + !periodic;
+          for (int J = 0; J < nc; ++J)
+            {
+              int    pos[ppf::restrict_taps<degree>];
+              double w[ppf::restrict_taps<degree>];
+              ppf::restrict_axis<degree>(J, nf, periodic, pos, w);
+              count(pos, w, nf, stray[0], outside[0]);
+            }
+          for (int I = 0; I < nf; ++I)
+            {
+              int    pos[degree + 1];
+              double w[degree + 1];
+              ppf::prolong_axis<degree>(I, nc, periodic, pos, w);
+              count(pos, w, nc, stray[1], outside[1]);
+            }
+        }
+    std::cout << "taps_q" << degree << ": " << stray[0] << " " << outside[0] << " " << stray[1]
+              << " " << outside[1] << "\n";
+  }
 } // namespace
 
 int
@@ -53,4 +97,6 @@ main()
             << refused(lattice(32768, 16385, 1), lattice(65536, 32769, 1))
             << refused(lattice(46341, 46340, 1), lattice(92681, 92679, 1)) << "\n"
             << "transfer_planes: " << refused(lattice(2, 2, 40000), lattice(3, 3, 79999)) << "\n";
+  transfer_taps<1>();
+  transfer_taps<2>();
 }

@@ -59,3 +59,10 @@ def test_transfer_launches_check_both_planes(logic):
     # The restriction runs over the coarse plane and reads the fine one with 32-bit indices.
     assert logic["transfer_fits"] == "00"
     assert logic["transfer_fine_plane"] == "1111" and logic["transfer_planes"] == "11"
+
+
+@pytest.mark.parametrize("degree", [1, 2])
+def test_transfers_read_only_what_their_outputs_take(logic, degree):
+    # Stray taps (weight zero, at a node the output does not depend on: 0 * NaN would reach
+    # it) and positions outside the lattice, of the restriction and of the prolongation.
+    assert logic[f"taps_q{degree}"] == "0 0 0 0"
