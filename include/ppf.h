@@ -114,7 +114,8 @@ int ppf_field_name(ppf_ctx *ctx, int field, char *buf, int len);
  * multigrid V-cycles that need no host synchronization are captured into a HIP graph
  * and replayed);
  * "synchronize" = 1|0 (0 leaves ppf_apply_operator asynchronous on the
- * context's stream); "write_output" = 0|1 (1: at every output increment ppf_run and
+ * context's stream; the first application of an operator on a stencil path waits all the
+ * same, to compare it with the generic path); "write_output" = 0|1 (1: at every output increment ppf_run and
  * ppf_solve_increment write the solution file of the `output` parameters,
  * <directory>/<file name>_<increment>.vtu, as SolutionOutput does, problem.cc:500-515);
  * "mg_level_precision" = double|single, "mg_coarse_solver" = smoother|cg,
@@ -181,6 +182,8 @@ int ppf_apply_operator(ppf_ctx *ctx, int block_id, int which, int scaling, int p
  * of PPF_NOALLOC_SCRATCH_BYTES per GPU and application library, held until the process
  * ends.  A launch that needs more fails with PPF_ERR_INVALID and a message naming the
  * size (e.g. the generic path needs fields x (degree+1)^dim x 8 B per cell in FP64).
+ * An elasticity-like operator whose stencil has not been compared with the generic path
+ * runs the latter while the comparison's reference (the block vector) does not fit.
  * Every call on a GPU shares that array: calls that overlap on one GPU (other threads,
  * other streams) race.  The context itself (ppf_create) still allocates as usual. */
 #define PPF_NOALLOC_SCRATCH_BYTES (64ll << 20)

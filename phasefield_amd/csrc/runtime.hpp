@@ -904,23 +904,24 @@ namespace ppf
       // plan is dropped (for good, with a line in the output log) if they disagree.  This
       // catches coefficients that branch on values or times the structure probe did not
       // visit.
+      bool in_place = false;
+      for (const number *d : dst)
+        for (const number *sp : src)
+          in_place = in_place || sp == d;
       if ((use_split || use_coupled) && path == OperatorPath::Auto && !entry.verified &&
-          lf.grid == &fine &&
-          !std::any_of(std::begin(dst), std::end(dst),
-                       [&](const number *d) {
-                         for (const number *sp : src)
-                           if (sp == d)
-                             return true;
-                         return false;
-                       }))
+          lf.grid == &fine && !in_place && !(use_coupled && capturing()))
         {
           const int64_t n   = g.n_nodes;
           number       *ref = nullptr;
           if (borrowed.base)
             {
+              // (the generic kernel of a coupled operator needs no scratch of its own)
+              const int64_t per_cell =
+                use_coupled ? 0
+                            : int64_t(bf.size()) * dofs_per_cell<dim, degree> * g.n_cells *
+                                  int64_t(sizeof(number)) + 256;
               if (borrowed.used + int64_t(bf.size()) * n * int64_t(sizeof(number)) + 256 +
-                    int64_t(bf.size()) * dofs_per_cell<dim, degree> * g.n_cells *
-                      int64_t(sizeof(number)) + 256 <=
+                    per_cell <=
                   borrowed.bytes)
                 ref = carve<number>(int64_t(bf.size()) * n, "the split-path comparison");
             }
@@ -993,7 +994,20 @@ namespace ppf
               return;
             }
         }
-      launch(use_split || use_coupled, out);
+      // A coupled plan that could not be compared (an operand in place, a stream under
+      // capture, too little borrowed scratch) leaves the application to the generic path that
+      // such operators always had.  (Levels have no comparison: their operators only
+      // precondition.)
+      launch(use_split || (use_coupled && (entry.verified || lf.grid != &fine)), out);
+    }
+
+    /// Whether the stream records a graph (no wait and no copy to the host is possible).
+    bool
+    capturing() const
+    {
+      hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+      PPF_HIP_CHECK(hipStreamIsCapturing(stream, &status));
+      return status != hipStreamCaptureStatusNone;
     }
 
     /// Whether the coupled stencil kernel runs a plan on lattice g: 3-D Q2, at least five

@@ -94,3 +94,75 @@ def test_coupled_stencil_matches_generic(device, mesh):
     slow.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, b.data_ptr())
     err = float(((a - b).abs() / b.abs()).max())
     assert err <= 1e-13, (mesh, err)
+
+
+def fresh_pair(cells, device, torch):
+    """A fresh context, one on the generic path, and a random block vector."""
+    text = mesh_text(cells, "", MIXED)
+    fast, slow = Context(APP, text), Context(APP, text)
+    slow.set_option("operator_path", "generic")
+    src = torch.tensor(np.random.default_rng(12).uniform(-1.0, 1.0, 3 * fast.info.n_nodes),
+                       device=device)
+    return fast, slow, src
+
+
+def test_first_application_can_be_captured(device):
+    """Nothing can be compared under capture: the generic kernel is recorded, and replays give
+    its bits whatever path eager applications in between take."""
+    import torch
+
+    fast, slow, src = fresh_pair((6, 5, 4), device, torch)
+    fast.set_option("synchronize", 0)
+    dst = torch.zeros_like(src)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.ExternalStream(fast.stream()),
+                          capture_error_mode="relaxed"):
+        fast.apply_operator(1, OP_LHS, SCALE_NONE, FP64, src.data_ptr(), dst.data_ptr())
+    for replay in range(4):
+        src.uniform_(-1.0, 1.0)
+        dst.fill_(7.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = apply(slow, torch, src, OP_LHS, SCALE_NONE, FP64)
+        assert np.array_equal(dst.cpu().numpy(), ref), replay
+        assert rel_err(apply(fast, torch, src, OP_LHS, SCALE_NONE, FP64), ref) <= 1e-13
+    assert "coupled stencil" in fast.output_log()
+
+
+def test_scratch_too_small_to_compare(device):
+    """142 x 142 x 142 nodes and more: the reference of the comparison does not fit the 64 MiB
+    of scratch, so an application without allocation runs the generic kernel until one with
+    allocation has checked the plan."""
+    import torch
+
+    fast, slow, src = fresh_pair((71, 71, 71), device, torch)
+    dst, ref = torch.empty_like(src), torch.empty_like(src)
+    args = (1, OP_LHS, SCALE_NONE, FP64, src.data_ptr())
+    slow.apply_operator(*args, ref.data_ptr())
+    fast.apply_operator_noalloc(*args, dst.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.equal(dst, ref) and "coupled stencil" not in fast.output_log()
+    fast.apply_operator(*args, dst.data_ptr())
+    assert "coupled stencil" in fast.output_log()
+    again = torch.empty_like(dst)
+    fast.apply_operator_noalloc(*args, again.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.equal(dst, again)
+    assert rel_err(dst.cpu().numpy(), ref.cpu().numpy()) <= 1e-13
+
+
+def test_small_scratch_compares(device):
+    """129 x 129 x 129 nodes: the reference fits, and the first application without
+    allocation checks the plan."""
+    import torch
+
+    fast, slow, src = fresh_pair((64, 64, 64), device, torch)
+    dst, ref = torch.empty_like(src), torch.empty_like(src)
+    args = (1, OP_LHS, SCALE_NONE, FP64, src.data_ptr())
+    slow.apply_operator(*args, ref.data_ptr())
+    fast.apply_operator_noalloc(*args, dst.data_ptr())
+    torch.cuda.synchronize()
+    assert "coupled stencil" in fast.output_log()
+    assert rel_err(dst.cpu().numpy(), ref.cpu().numpy()) <= 1e-13
