@@ -100,6 +100,26 @@ namespace ppf
     }
   };
 
+  /// What the comparison of a plan's result with the generic path's says, from the largest
+  /// difference and the largest reference value.
+  enum class PlanCheck
+  {
+    Agrees,
+    Differs,
+    Undecided ///< compare again at the next application
+  };
+
+  /// Zero against zero says nothing of a coupled plan's coefficients (a solve from zero begins
+  /// with such an application).  Plans of the split path have always been taken then: fields at
+  /// rest would be compared in every increment.
+  inline PlanCheck
+  check_plan(const SplitPlan &plan, double worst, double scale, double tol)
+  {
+    if (scale == 0.0 && worst == 0.0)
+      return plan.coupled ? PlanCheck::Undecided : PlanCheck::Agrees;
+    return worst <= tol * scale ? PlanCheck::Agrees : PlanCheck::Differs;
+  }
+
   template <class PDE, int dim, int degree, typename number>
   class HookProbe
   {

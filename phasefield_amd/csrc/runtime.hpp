@@ -971,9 +971,10 @@ namespace ppf
                                         hipMemcpyDeviceToHost));
               if (!halted_now)
                 {
-                  const double tol = std::is_same_v<number, float> ? 1e-4 : 1e-11;
-                  entry.verified   = true;
-                  if (!(worst <= tol * scale) && !(scale == 0.0 && worst == 0.0))
+                  const double    tol   = std::is_same_v<number, float> ? 1e-4 : 1e-11;
+                  const PlanCheck check = check_plan(plan, worst, scale, tol);
+                  entry.verified        = check != PlanCheck::Undecided;
+                  if (check == PlanCheck::Differs)
                     {
                       std::ostringstream msg;
                       msg << "solve block " << blk.id << " (" << (lhs ? "lhs" : "rhs")
@@ -983,6 +984,7 @@ namespace ppf
                       entry.plan.eligible = false;
                       entry.plan.coupled  = false;
                       entry.plan.reason   = msg.str();
+                      ++graph_epoch; // captured V-cycles may launch the dropped path
                       log += msg.str() + "\n";
                       if (std::getenv("PPF_VERBOSE"))
                         std::fprintf(stderr, "%s\n", msg.str().c_str());

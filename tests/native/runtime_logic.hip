@@ -1,8 +1,11 @@
 // Prints host evaluations of functions that the kernels and their launches share.
+#include "operator_plan.hpp"
 #include "vector_kernels.hpp"
 
 #include <iostream>
+#include <limits>
 #include <string>
+#include <utility>
 
 namespace
 {
@@ -97,6 +100,19 @@ main()
             << refused(lattice(32768, 16385, 1), lattice(65536, 32769, 1))
             << refused(lattice(46341, 46340, 1), lattice(92681, 92679, 1)) << "\n"
             << "transfer_planes: " << refused(lattice(2, 2, 40000), lattice(3, 3, 79999)) << "\n";
+  // comparisons: in agreement, apart, zero with zero, nothing with something, not finite
+  for (bool coupled : {false, true})
+    {
+      ppf::SplitPlan plan;
+      plan.eligible = !coupled;
+      plan.coupled  = coupled;
+      std::cout << (coupled ? "check_coupled: " : "check_split: ");
+      const double inf = std::numeric_limits<double>::infinity();
+      for (auto [worst, scale] : {std::pair {1e-13, 2.0}, {1e-3, 2.0}, {0.0, 0.0}, {1e-30, 0.0},
+                                  {inf, 2.0}, {inf, 0.0}})
+        std::cout << int(ppf::check_plan(plan, worst, scale, 1e-11));
+      std::cout << "\n";
+    }
   transfer_taps<1>();
   transfer_taps<2>();
 }

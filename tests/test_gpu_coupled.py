@@ -166,3 +166,21 @@ def test_small_scratch_compares(device):
     torch.cuda.synchronize()
     assert "coupled stencil" in fast.output_log()
     assert rel_err(dst.cpu().numpy(), ref.cpu().numpy()) <= 1e-13
+
+
+def test_zero_operand_checks_nothing(device):
+    """An application to zero agrees whatever the coefficients are: the inverse diagonal is
+    probed on the generic path (its bits) until an application to something has agreed."""
+    import torch
+
+    fast, slow, src = fresh_pair((6, 5, 4), device, torch)
+    diag, ref = torch.empty_like(src), torch.empty_like(src)
+    slow.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, ref.data_ptr())
+    for _ in range(2):
+        assert not apply(fast, torch, torch.zeros_like(src), OP_LHS, SCALE_NONE, FP64).any()
+        fast.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, diag.data_ptr())
+        assert torch.equal(diag, ref)
+    apply(fast, torch, src, OP_LHS, SCALE_NONE, FP64)
+    fast.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, diag.data_ptr())
+    assert not torch.equal(diag, ref)  # from the coefficients
+    assert float(((diag - ref).abs() / ref.abs()).max()) <= 1e-13

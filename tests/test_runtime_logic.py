@@ -66,3 +66,9 @@ def test_transfers_read_only_what_their_outputs_take(logic, degree):
     # Stray taps (weight zero, at a node the output does not depend on: 0 * NaN would reach
     # it) and positions outside the lattice, of the restriction and of the prolongation.
     assert logic[f"taps_q{degree}"] == "0 0 0 0"
+
+
+def test_comparison_of_zero_with_zero_checks_no_coupled_plan(logic):
+    # 0 agrees, 1 differs, 2 undecided
+    assert logic["check_split"] == "010111"
+    assert logic["check_coupled"] == "012111"
