@@ -120,6 +120,14 @@ namespace ppf
     return worst <= tol * scale ? PlanCheck::Agrees : PlanCheck::Differs;
   }
 
+  /// Whether a plan derived anew (another time step, time or increment) keeps the comparison of
+  /// the one before: it does if the same path takes the operator.
+  inline bool
+  keeps_check(const SplitPlan &before, const SplitPlan &now)
+  {
+    return now.stencil() && now.eligible == before.eligible && now.coupled == before.coupled;
+  }
+
   template <class PDE, int dim, int degree, typename number>
   class HookProbe
   {

@@ -708,7 +708,7 @@ namespace ppf
           entry.verified      = true;
         }
       else if (it != plans.end())
-        entry.verified = it->second.verified && entry.plan.stencil();
+        entry.verified = it->second.verified && keeps_check(it->second.plan, entry.plan);
       return plans[key] = entry, plans[key];
     }
 

@@ -113,6 +113,19 @@ main()
         std::cout << int(ppf::check_plan(plan, worst, scale, 1e-11));
       std::cout << "\n";
     }
+  // plans derived anew: split, coupled and generic before, each followed by each
+  std::cout << "keeps_check: ";
+  for (int before = 0; before < 3; ++before)
+    for (int now = 0; now < 3; ++now)
+      {
+        ppf::SplitPlan p, q;
+        p.eligible = before == 0;
+        p.coupled  = before == 1;
+        q.eligible = now == 0;
+        q.coupled  = now == 1;
+        std::cout << ppf::keeps_check(p, q);
+      }
+  std::cout << "\n";
   transfer_taps<1>();
   transfer_taps<2>();
 }

@@ -72,3 +72,7 @@ def test_comparison_of_zero_with_zero_checks_no_coupled_plan(logic):
     # 0 agrees, 1 differs, 2 undecided
     assert logic["check_split"] == "010111"
     assert logic["check_coupled"] == "012111"
+
+
+def test_comparison_is_kept_by_the_same_path_only(logic):
+    assert logic["keeps_check"] == "100" "010" "000"
