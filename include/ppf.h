@@ -101,9 +101,12 @@ int ppf_field_name(ppf_ctx *ctx, int field, char *buf, int len);
  * kernel, split_node: one thread per node); "stencil_waves" = 0|4|8,
  * "stencil_rows" = 0|1|2|4 (waves x rows: 4x2, 4x4, 8x1 or 8x2) and
  * "stencil_z_chunk" = <planes> (0: automatic) tune the tiled kernel's workgroup
- * shape; "stencil_min_nodes" = <n>: lattices with fewer
- * nodes run split operators column by column instead of by tiles, those with two stencil
- * operands node by node (defaults 1000000, in 2-D 500000, and 100000; 0: tiles at any size); "stencil_store_policy" = auto|temporal|nontemporal sets the cache policy of
+ * shape, "stencil_map" = auto|linear|band the order of its workgroups (auto: a band of
+ * tile rows per XCD on 3-D lattices of 4 M nodes and more); "stencil_min_nodes" = auto|<n>:
+ * lattices with fewer nodes run split operators column by column instead of by tiles, those
+ * with two stencil operands node by node (auto: 1000000, in 2-D 500000, and 100000; both
+ * 100000 while one of the four options before is set; 0: tiles at any size);
+ * "stencil_store_policy" = auto|temporal|nontemporal sets the cache policy of
  * its output stores (auto: non-temporal when the launch's arrays exceed 512 MiB);
  * "generic_kernel" = cell_block|two_pass selects the generic path's kernels (cell_block:
  * one launch, cell blocks staged in shared memory, no device scratch; two_pass: a cell

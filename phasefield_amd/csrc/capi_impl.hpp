@@ -359,9 +359,9 @@ ppf_set_option(ppf_ctx *ctx, const char *key, const char *value)
       c.rt.stencil_z_chunk = std::stoi(v);
     else if (k == "stencil_map")
       {
-        if (v != "linear" && v != "band")
-          throw ppf::Error(ppf::status_invalid, "stencil_map: linear or band");
-        c.rt.stencil_map = v == "band" ? 1 : 0;
+        if (v != "auto" && v != "linear" && v != "band")
+          throw ppf::Error(ppf::status_invalid, "stencil_map: auto, linear or band");
+        c.rt.stencil_map = v == "auto" ? -1 : (v == "band" ? 1 : 0);
       }
     else if (k == "generic_kernel")
       {
@@ -378,7 +378,7 @@ ppf_set_option(ppf_ctx *ctx, const char *key, const char *value)
         c.rt.mg_graphs = v == "1";
       }
     else if (k == "stencil_min_nodes")
-      c.rt.stencil_min_nodes = std::max<int64_t>(0, std::stoll(v));
+      c.rt.stencil_min_nodes = v == "auto" ? -1 : std::max<int64_t>(0, std::stoll(v));
     else if (k == "stencil_target_blocks")
       c.rt.stencil_target_blocks = std::max(1, std::stoi(v));
     else if (k == "stencil_store_policy")

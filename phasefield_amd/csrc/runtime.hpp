@@ -4245,24 +4245,21 @@ namespace ppf
     /// launches whose arrays exceed stencil_nt_min_bytes).
     StorePolicy                            stencil_store_policy = StorePolicy::Auto;
     int64_t                                stencil_nt_min_bytes = int64_t(512) << 20;
-    /// Lattices with fewer nodes run split operators column by column (two stencil
-    /// operands: node by node) instead of by marching tiles (launch_stencil).  Measured per
-    /// increment or application, tile / column: Cahn-Hilliard Q2 (periodic) 110k nodes 26.7 /
-    /// 17.9 us, 885k 29.3 / 25.5, 1.4M 30.6 / 32.8; precipitate Q1 885k 37.1 / 30.6, 2.1M 46.0
-    /// / 46.1; Poisson Q2 (Dirichlet) 531k FP64 13.9 / 12.9, FP32 12.3 / 10.6, 1.5M 16.3 / 20.0.
-    /// In 2-D (Allen-Cahn Q1) 250k nodes 7.0 / 6.9, 490k 7.19 / 7.17, 790k 8.55 / 8.93.
-    /// The node kernel's limit is older: BiCGStab on two operands stops on the last bits of
-    /// its sums, so those lattices keep their kernels.  Option stencil_min_nodes sets both.
+    /// Lattices with fewer nodes run split operators column by column, with two stencil
+    /// operands node by node, instead of by marching tiles (launch_stencil): option
+    /// stencil_min_nodes sets both limits (-1: by size, column_limit and node_limit).
     int64_t                                stencil_min_nodes    = -1;
     int64_t
     column_kernel_limit() const
     {
-      return stencil_min_nodes < 0 ? (dim == 3 ? 1000000 : 500000) : stencil_min_nodes;
+      return column_limit(dim, stencil_min_nodes,
+                          stencil_waves != 0 || stencil_rows != 0 || stencil_z_chunk != 0 ||
+                            stencil_map >= 0);
     }
     int64_t
     node_kernel_limit() const
     {
-      return stencil_min_nodes < 0 ? 100000 : stencil_min_nodes;
+      return node_limit(stencil_min_nodes);
     }
     /// Start every linear solve from zero instead of the previous solution (which the
     /// reference keeps as the next initial guess, linear_solver.h:330-336).

@@ -756,6 +756,32 @@ namespace ppf
       run(std::integral_constant<bool, false> {});
   }
 
+  /// Lattices with fewer nodes take split operators of two stencil operands node by node.
+  /// (Older than the column kernel: BiCGStab on two operands stops on the last bits of its
+  /// sums, so those lattices keep their kernels.)  min_nodes: set by the program, or -1.
+  inline int64_t
+  node_limit(int64_t min_nodes)
+  {
+    return min_nodes < 0 ? 100000 : min_nodes;
+  }
+
+  /// Lattices with fewer nodes take split operators of at most one stencil operand column by
+  /// column.  Measured per increment or application, tile / column: Cahn-Hilliard Q2 (periodic)
+  /// 110k nodes 26.7 / 17.9 us, 885k 29.3 / 25.5, 1.4M 30.6 / 32.8; precipitate Q1 885k 37.1 /
+  /// 30.6, 2.1M 46.0 / 46.1; Poisson Q2 (Dirichlet) FP64 531k 10.6 / 9.5, 913k 12.2 / 11.2, 1.16M
+  /// 12.4 / 13.3, 2.15M 15.1 / 19.5; FP32 913k 9.6 / 8.5, 1.16M 9.7 / 9.3, 1.44M 9.8 / 10.1, 2.78M
+  /// 11.4 / 15.0 (half the bytes, but about the same line: the column kernel issues ten loads
+  /// per node in either type).  In 2-D (Allen-Cahn Q1) 250k nodes 7.0 / 6.9, 490k 7.19 / 7.17,
+  /// 790k 8.55 / 8.93.  A program that sets the tiles' shape or order (`tiles_set`) gets tiles
+  /// from node_limit on.
+  inline int64_t
+  column_limit(int dim, int64_t min_nodes, bool tiles_set)
+  {
+    if (min_nodes >= 0 || tiles_set)
+      return node_limit(min_nodes);
+    return dim == 3 ? 1000000 : 500000;
+  }
+
   /// Planes a thread of stencil_column_kernel owns.
   template <int dim>
   constexpr int stencil_column_planes = dim == 3 ? 4 : 1;

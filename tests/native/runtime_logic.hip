@@ -1,5 +1,6 @@
 // Prints host evaluations of functions that the kernels and their launches share.
 #include "operator_plan.hpp"
+#include "stencil_kernels.hpp"
 #include "vector_kernels.hpp"
 
 #include <iostream>
@@ -126,6 +127,12 @@ main()
         std::cout << ppf::keeps_check(p, q);
       }
   std::cout << "\n";
+  std::cout << "limits_auto: " << ppf::column_limit(2, -1, false) << " "
+            << ppf::column_limit(3, -1, false) << " " << ppf::node_limit(-1) << "\n"
+            << "limits_tiles: " << ppf::column_limit(2, -1, true) << " "
+            << ppf::column_limit(3, -1, true) << "\n"
+            << "limits_given: " << ppf::column_limit(3, 0, true) << " "
+            << ppf::column_limit(3, 7, false) << " " << ppf::node_limit(7) << "\n";
   transfer_taps<1>();
   transfer_taps<2>();
 }

@@ -557,3 +557,13 @@ def test_solution_files_at_output_increments(device, tmp_path):
     for f, name in enumerate(("n", "f_tot")):
         np.testing.assert_array_equal(arrs[name], ctx.get_field(f, AGE_LATEST).ravel())
     assert arrs["CYCLE"][0] == 4
+
+
+def test_automatic_tile_options_can_be_restored(device):
+    ctx = Context("cahn_hilliard_3d_q2", prm.cahn_hilliard(refinement=2))
+    for key, values in {"stencil_map": ("band", "linear", "auto"),
+                        "stencil_min_nodes": ("0", "1000", "auto")}.items():
+        for value in values:
+            ctx.set_option(key, value)
+        with pytest.raises(PPFError):
+            ctx.set_option(key, "automatic")

@@ -76,3 +76,10 @@ def test_comparison_of_zero_with_zero_checks_no_coupled_plan(logic):
 
 def test_comparison_is_kept_by_the_same_path_only(logic):
     assert logic["keeps_check"] == "100" "010" "000"
+
+
+def test_tile_options_reach_the_tiles(logic):
+    assert logic["limits_auto"] == "500000 1000000 100000"
+    # a tile shape or order that is set acts from where it did before the column kernel
+    assert logic["limits_tiles"] == "100000 100000"
+    assert logic["limits_given"] == "0 7 7"
