@@ -13,8 +13,9 @@ namespace ppf
     unsigned int word;
   };
 
-  /// Tags of the scalars and the entries they go to.  At most two scalars are under way at a
-  /// time, so an entry is read before it is issued again.
+  /// Tags of the scalars and the entries they go to.  At most four scalars are under way at a
+  /// time (the residual of a CG step, the two maxima of a plan compared in the step enqueued
+  /// ahead, and that step's residual), so an entry is read before it is issued again.
   class HostScalarRing
   {
   public:

@@ -64,13 +64,22 @@ namespace ppf
     return r;
   }
 
-  /// Per-block max |a - b| (NaN or infinite counted as +inf) and max |b|, into
-  /// partial[b] and partial[gridDim.x + b].
+  /// Vectors to compare: one pair per field of a block.
+  template <typename T>
+  struct ComparedFields
+  {
+    const T *a[PPF_MAX_FIELDS];
+    const T *b[PPF_MAX_FIELDS];
+  };
+
+  /// Per-block max |a - b| (NaN or infinite counted as +inf) and max |b| of a field, into
+  /// partial[i] and partial[all + i] for block i of all.  Grid: x over the vectors, y the fields.
   template <typename T>
   __global__ void __launch_bounds__(reduce_threads)
-  max_diff_partial_kernel(double *__restrict__ partial, const T *__restrict__ a,
-                          const T *__restrict__ b, int64_t n)
+  max_diff_partial_kernel(double *__restrict__ partial, const ComparedFields<T> f, int64_t n)
   {
+    const T *__restrict__ a = f.a[blockIdx.y];
+    const T *__restrict__ b = f.b[blockIdx.y];
     double d = 0.0, m = 0.0;
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
          i += int64_t(gridDim.x) * blockDim.x)
@@ -84,8 +93,9 @@ namespace ppf
     m = block_max(m);
     if (threadIdx.x == 0)
       {
-        partial[blockIdx.x]             = d;
-        partial[gridDim.x + blockIdx.x] = m;
+        const int i = int(blockIdx.x + gridDim.x * blockIdx.y);
+        partial[i]  = d;
+        partial[int(gridDim.x * gridDim.y) + i] = m;
       }
   }
 
@@ -388,6 +398,27 @@ namespace ppf
     const double s = sum_partials(partial, count);
     if (threadIdx.x == 0)
       tell_host(to, s, tag, false);
+  }
+
+  /// Tells the host the maxima of both halves of 2 * count partials; launched as one workgroup.
+  __global__ void __launch_bounds__(reduce_threads)
+  max_to_host_kernel(HostScalar *first, unsigned int first_tag, HostScalar *second,
+                     unsigned int second_tag, const double *__restrict__ partial, int count)
+  {
+    double d = 0.0, m = 0.0;
+    for (int i = threadIdx.x; i < count; i += reduce_threads)
+      {
+        d = fmax(d, partial[i]);
+        m = fmax(m, partial[count + i]);
+      }
+    d = block_max(d);
+    __syncthreads();
+    m = block_max(m);
+    if (threadIdx.x == 0)
+      {
+        tell_host(first, d, first_tag, false);
+        tell_host(second, m, second_tag, false);
+      }
   }
 
   /// Per-block partial sums of x.y; nothing once *done is set (done may be null).
