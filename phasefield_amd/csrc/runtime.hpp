@@ -1423,12 +1423,9 @@ namespace ppf
       // 32-bit byte offsets in the kernel: arrays up to 4 GiB.
       if (int64_t(a.n[0]) * a.n[1] * a.n[2] * int64_t(sizeof(ST)) > (int64_t(1) << 32))
         return false;
-      // Store policy: non-temporal when the distinct arrays the launch reads and writes
-      // exceed twice the 256 MB Infinity Cache, so that none of the output would still be
-      // there for the launch that reads it.  Below that the consumer pays for it: four Poisson
-      // applications at 257^3 nodes (FP64, 271 MB each), each reading the one before, take 75
-      // us per application with temporal and 83 us with non-temporal stores (repeated on one
-      // unread output: 69 and 62 us); the Cahn-Hilliard increment at 129^3 31.3 and 33.4 us.
+      // Store policy: non-temporal when the distinct arrays the launch reads and writes exceed
+      // the 256 MB Infinity Cache (stencil_nt_min_bytes): beyond it the output would not be
+      // there for the launch that reads it.
       {
         const void *arrays[stencil_max_ops + PPF_MAX_FIELDS * (PPF_N_SLOTS + 1)];
         int         n_arrays = 0;
@@ -4246,10 +4243,17 @@ namespace ppf
     int64_t                                n_cus_     = 0;
     int64_t                                lds_limit_ = 0;
     int                                    stencil_target_blocks = 2048;
-    /// Cache policy of the stencil kernel's output stores (Auto: non-temporal for
-    /// launches whose arrays exceed stencil_nt_min_bytes).
+    /// Cache policy of the stencil kernel's output stores (Auto: non-temporal for launches
+    /// whose arrays exceed stencil_nt_min_bytes, the size of the Infinity Cache).  Measured,
+    /// temporal / non-temporal, launches that read each other's output, by the bytes of a
+    /// launch: four Poisson Q2 applications (FP64) 214 MiB 53.9 / 61.5 us each, 259 MiB 71.5 /
+    /// 73.0, 284 MiB 91.1 / 90.6, 368 MiB 112 / 109; the coupled stencil 254 MiB 94.3 / 99.2, 329
+    /// MiB 121.5 / 121.9.  Increments, by the line drawn at 192 / 256 / 384 MiB: Cahn-Hilliard
+    /// 104^3 cells 105.7 / 90.4 / 90.1 us, 128^3 141.1 / 136.4 / 154.6; precipitate 224^3 168.6 /
+    /// 168.4 / 192.5, 256^3 218 / 218 / 247.5, 192^3 the same.  An output that nothing reads next is
+    /// better stored non-temporally above 230 MiB: 259 MiB 65.4 / 62.1, 310 MiB 91.6 / 66.5.
     StorePolicy                            stencil_store_policy = StorePolicy::Auto;
-    int64_t                                stencil_nt_min_bytes = int64_t(512) << 20;
+    int64_t                                stencil_nt_min_bytes = int64_t(256) << 20;
     /// Lattices with fewer nodes run split operators column by column, with two stencil
     /// operands node by node, instead of by marching tiles (launch_stencil): option
     /// stencil_min_nodes sets both limits (-1: by size, column_limit and node_limit).
