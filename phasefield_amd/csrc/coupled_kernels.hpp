@@ -5,8 +5,9 @@
 //
 //   t[c][d] = sum_{s,e} C[c][d][s][e] du_s/dx_e
 //
-// with constants C, no value term and the coupling of an orthotropic material assembles on the uniform GLL-collocated Q2 mesh to
-// sums of tensor products of 1-D matrices, because the quadrature points are the nodes:
+// with constants C, no value term and the coupling of an orthotropic material assembles on
+// the uniform GLL-collocated Q2 mesh to sums of tensor products of 1-D matrices, because the
+// quadrature points are the nodes:
 //
 //   d = e: K_d (stiffness) times the lumped masses of the other axes;
 //   d != e: G_d^T G_e times the lumped mass of the third axis, G = assembled (w_i D_ij).
@@ -442,9 +443,9 @@ namespace ppf
       }
   }
 
-  /// Diagonal of the same operator: M_i^scaling (sum_d C[c][d][c][d] L_d(0) + sum_{d != e}
-  /// C[c][d][c][e] (g_d^T)(0) g_e(0)); the mixed products are nonzero only where two
-  /// boundary faces meet.  Inverted as invert_diagonal_kernel does.
+  /// Diagonal of the same operator: M_i^scaling sum_d C[c][d][c][d] L_d(0).  (Mixed
+  /// derivatives couple different components only, see orthotropic_term.)  Inverted as
+  /// invert_diagonal_kernel does.
   template <typename number>
   __global__ void __launch_bounds__(block_size)
   coupled_inverse_diagonal_kernel(const GridDesc g, const CoupledArgs<number> a, int c,
@@ -460,18 +461,9 @@ namespace ppf
         inv[node] = number(1);
         return;
       }
-    double g0[3], t0[3], k = 0.0;
+    double k = 0.0;
     for (int d = 0; d < 3; ++d)
-      {
-        double t[5];
-        derivative_taps(i[d], g.nodes[d], g.periodic[d], t);
-        g0[d] = t[2];
-        t0[d] = t[2] == 0.0 ? 0.0 : -t[2] + (t[2] < 0.0 ? -6.0 : 6.0);
-        k += double(a.coef[c][d][c]) * ((i[d] & 1) ? 8.0 : 14.0);
-      }
-    const int de[6][2] = {{0, 1}, {0, 2}, {1, 0}, {1, 2}, {2, 0}, {2, 1}};
-    for (int m = 0; m < 6; ++m)
-      k += double(a.coef[c][6 + m][c]) * t0[de[m][0]] * g0[de[m][1]];
+      k += double(a.coef[c][d][c]) * ((i[d] & 1) ? 8.0 : 14.0);
     const double v = node_scaling<3, 2>(g, i, scaling) * lumped_mass<3, 2>(g, i) * k;
     inv[node]      = number(v) == number(0) ? number(1) : number(1) / number(v);
   }

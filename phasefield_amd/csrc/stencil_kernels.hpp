@@ -168,18 +168,6 @@ namespace ppf
     return (degree == 2 && (i & 1)) ? 0 : 1;
   }
 
-  /// Node class of the inverse-diagonal tables along one axis (axis_class).
-  template <int degree>
-  PPF_HD PPF_INLINE int
-  line_class(int i, int n, int periodic)
-  {
-    if (!periodic && i == 0)
-      return 2;
-    if (!periodic && i == n - 1)
-      return 3;
-    return (degree == 2 && (i & 1)) ? 0 : 1;
-  }
-
   /// Host-side 1-D lumped mass of scale class c, in units of h.
   template <int degree>
   inline double
@@ -787,12 +775,14 @@ namespace ppf
   constexpr int stencil_column_planes = dim == 3 ? 4 : 1;
   constexpr int stencil_column_threads = 256;
 
-  /// The same operator, with at most one stencil operand, without tiles: a thread owns one (x, y) column of a few planes, the
-  /// threads of a workgroup consecutive nodes of the flattened x-y plane (no lane is idle
-  /// at a ragged width).  Every operand value comes from the caches through a load of its
-  /// own, all of them issued before the first is used: there is no march, so the time of a
-  /// launch is about one memory latency plus the issue of 9 (Q1: 6) loads per node, where
-  /// a tile of stencil_operator_kernel waits once per plane.  Same arithmetic, same bits.
+  /// The same operator, with at most one stencil operand, without tiles: a thread owns one
+  /// (x, y) column of a few planes, the threads of a workgroup consecutive nodes of the
+  /// flattened x-y plane (no lane is idle at a ragged width).  Every operand value comes from
+  /// the caches through a load of its own, all of them issued before the first is used: there is
+  /// no march, so the time of a launch is about one memory latency plus the issue of 10 (Q1:
+  /// 5.5) loads per node, where a tile of stencil_operator_kernel waits once per plane.  The
+  /// stencil's sums have the tiles' order and bits; the compiler may contract a hook's own
+  /// products differently here (seen with FP32 arithmetic, 1e-8 of the result).
   ///
   /// a.tiles_x: workgroups per plane, a.chunks_z: plane groups, a.n_blocks: their product.
   /// MASKED: some operand, input or output has Dirichlet faces.
@@ -992,9 +982,9 @@ namespace ppf
                 const ST r = sm_b[k] - (dir ? ST(0) : ST(scale * acc));
                 const unsigned int i = q + unsigned(z) * (unsigned(n0) * unsigned(n1));
                 const ST inv = sm.table && *sm.ok
-                                 ? sm.table[line_class<degree>(x, n0, p0) +
-                                            4 * line_class<degree>(y, n1, p1) +
-                                            16 * (dim == 3 ? line_class<degree>(z, n2, p2) : 1)]
+                                 ? sm.table[line_class(degree, x, n0, p0) +
+                                            4 * line_class(degree, y, n1, p1) +
+                                            16 * (dim == 3 ? line_class(degree, z, n2, p2) : 1)]
                                  : sm.inv_diag[i];
                 const ST d = sm.first ? sm.c2 * inv * r : sm.c1 * sm_d[k] + sm.c2 * inv * r;
                 buffer_store(d, make_rsrc(sm.d), own, po, false);

@@ -643,19 +643,21 @@ namespace ppf
 
   constexpr int diag_classes = 64;
 
+  /// Node class of the inverse-diagonal tables along one axis of n nodes.
+  PPF_HD PPF_INLINE int
+  line_class(int degree, int i, int n, int periodic)
+  {
+    if (!periodic && i == 0)
+      return 2;
+    if (!periodic && i == n - 1)
+      return 3;
+    return (degree == 2 && (i & 1)) ? 0 : 1;
+  }
+
   PPF_HD PPF_INLINE int
   axis_class(const ClassGrid &g, int d, int i)
   {
-    if (d >= g.dim)
-      return 1;
-    if (!g.periodic[d])
-      {
-        if (i == 0)
-          return 2;
-        if (i == g.n[d] - 1)
-          return 3;
-      }
-    return (g.degree == 2 && (i & 1)) ? 0 : 1;
+    return d < g.dim ? line_class(g.degree, i, g.n[d], g.periodic[d]) : 1;
   }
 
   /// Representative coordinate of class c along axis d, -1 if the class does not occur.
@@ -937,7 +939,6 @@ namespace ppf
   template <int degree>
   constexpr int restrict_taps = degree == 1 ? 3 : 5;
 
-  template <int degree>
   PPF_HD constexpr int
   restrict_offset(int k)
   {
@@ -964,7 +965,7 @@ namespace ppf
 #pragma unroll
     for (int k = 0; k < restrict_taps<degree>; ++k)
       {
-        int  i  = 2 * J + restrict_offset<degree>(k);
+        int  i  = 2 * J + restrict_offset(k);
         bool ok = true;
         if (periodic) // a finer periodic lattice has at least 2 cells: one wrap suffices
           i = i < 0 ? i + n : (i >= n ? i - n : i);
@@ -1065,7 +1066,7 @@ namespace ppf
                 for (int j = 0; j < ZC; ++j)
 #pragma unroll
                   for (int k = 0; k < K; ++k)
-                    if (restrict_offset<degree>(k) == t - 2 * j &&
+                    if (restrict_offset(k) == t - 2 * j &&
                         restrict_weight<degree>(k, j % 2 == 0) != 0.0)
                       acc[j] = fma(T(restrict_weight<degree>(k, j % 2 == 0)), s, acc[j]);
               }
