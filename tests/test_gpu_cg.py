@@ -39,3 +39,22 @@ def test_cg_stops_like_the_oracle(device, oracle_libs, refinement, limit, precon
     st, ref = ctx.linear_solve(1), orc.linear_solve(1)
     assert st.iterations == ref["iterations"]
     assert rel_err(ctx.get_field(0, AGE_LATEST).ravel(), orc.get_field(0, AGE_LATEST)) <= 1e-9
+
+
+@pytest.mark.parametrize("cells, workgroups", [((255, 256), 1024), ((256, 256), 1029),
+                                               ((300, 300), 1411)])
+def test_cg_around_the_limit_of_partial_sums(device, oracle_libs, cells, workgroups):
+    """2-D lattices of the column kernel on both sides of 1024 workgroups, the partial sums that
+    d.Ad of the operator's own launch has room for: 511 x 513, 513 x 513 and 601 x 601 nodes.
+    The solve is cut short: the iterates of 25 steps are compared (condition number 1e5)."""
+    text = prm.poisson(dim=2, refinement=0, subdivisions=list(cells), mg_depth=1, tolerance=1e-9,
+                       preconditioner="None", max_iterations=25)
+    ctx, orc = Context("poisson_2d_q2", text), Oracle("poisson_2d_q2", text)
+    assert (ctx.info.n_nodes + 255) // 256 == workgroups
+    for c in (ctx, orc):
+        c.solve_block(0)
+        c.set_time(1, 0.0)
+    for _ in range(2):  # from zero, then on from there
+        st, ref = ctx.linear_solve(1), orc.linear_solve(1)
+        assert st.iterations == ref["iterations"] == 25
+        assert rel_err(ctx.get_field(0, AGE_LATEST).ravel(), orc.get_field(0, AGE_LATEST)) <= 1e-9
