@@ -12,10 +12,10 @@ struct Switching2D
 {
   static constexpr int dim      = 2;
   static constexpr int degree   = 2;
-  static constexpr int n_fields = 4;
+  static constexpr int n_fields = 5;
   template <typename number>
   using PDE      = prismspf::CustomPDE<dim, degree, number>;
-  using BlockIds = std::integer_sequence<int, 0, 1, 2, 3>;
+  using BlockIds = std::integer_sequence<int, 0, 1, 2, 3, 4>;
 
   static const char *
   name()

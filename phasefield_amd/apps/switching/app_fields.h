@@ -1,4 +1,5 @@
-// Fields and solve blocks of the routing test bed (four explicit diffusion blocks).
+// Fields and solve blocks of the routing test bed (four explicit diffusion blocks
+// and a linear one).
 #pragma once
 
 #include <prismspf/core/dependencies.h>
@@ -15,7 +16,7 @@ switching_define(std::vector<prismspf::FieldAttributes> &fields,
 {
   using namespace prismspf;
   fields = {FieldAttributes("c"), FieldAttributes("s"), FieldAttributes("r"),
-            FieldAttributes("u")};
+            FieldAttributes("u"), FieldAttributes("w")};
   auto block = [&](Types::Index id, std::set<std::string> deps) {
     SolveBlock b;
     b.id               = id;
@@ -25,8 +26,15 @@ switching_define(std::vector<prismspf::FieldAttributes> &fields,
     b.dependencies_rhs = make_dependency_set(fields, deps);
     return b;
   };
+  SolveBlock linear;
+  linear.id               = 4;
+  linear.solve_type       = Linear;
+  linear.solve_timing     = Primary;
+  linear.field_indices    = {4};
+  linear.dependencies_rhs = make_dependency_set(fields, {"c"});
+  linear.dependencies_lhs = make_dependency_set(fields, {"c", "lhs(w)", "grad(lhs(w))"});
   blocks = {block(0, {"old_1(c)", "grad(old_1(c))"}),
             block(1, {"old_1(c)", "old_1(s)", "grad(old_1(s))"}),
             block(2, {"old_1(r)", "grad(old_1(r))"}),
-            block(3, {"old_1(c)", "old_1(u)", "grad(old_1(u))"})};
+            block(3, {"old_1(c)", "old_1(u)", "grad(old_1(u))"}), linear};
 }

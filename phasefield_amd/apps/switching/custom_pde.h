@@ -1,6 +1,6 @@
 // Test-bed equations for the routing of hooks between the split (stencil) path and the
-// generic cell path, written against PRISMS-PF's application API.  Three explicit
-// diffusion blocks whose flux coefficients are constant on some inputs only:
+// generic cell path, written against PRISMS-PF's application API.  Explicit diffusion blocks
+// and a linear one whose flux coefficients are constant on some inputs only:
 //
 //   block 0 (c): value c_old, gradient -dt D grad(c_old)             (constant: split)
 //   block 1 (s): value s_old, gradient -dt D b(c_old) grad(s_old),
@@ -10,6 +10,9 @@
 //   block 3 (u): value u_old, gradient -dt D e(c_old) grad(u_old),
 //                e = 1 for c_old <= 60, 2 above                        (value branch
 //                                                                       beyond the probe)
+//   block 4 (w): linear, value w, gradient D e(c) grad(w), right-hand side c / 50
+//                                                                      (the same branch in
+//                                                                       a solve's operator)
 //
 // Model constants: D, c_low, c_high (the initial c ramps from c_low at x = 0 to c_high).
 #include <prismspf/core/pde_operator_base.h>
@@ -90,6 +93,26 @@ private:
           c, ScalarValue(60.0), ScalarValue(2.0), ScalarValue(1.0));
         variable_list.set_value_term(3, u);
         variable_list.set_gradient_term(3, -dt * D * e * ux);
+      }
+    else if (solve_block_id == 4)
+      variable_list.set_value_term(
+        4, ScalarValue(0.02) * variable_list.template get_value<Scalar, Current>(0));
+  }
+
+  void
+  compute_lhs(FieldContainer<dim, degree, number> &variable_list,
+              [[maybe_unused]] const SimulationTimer &sim_timer,
+              unsigned int                             solve_block_id) const override
+  {
+    if (solve_block_id == 4)
+      {
+        ScalarValue c  = variable_list.template get_value<Scalar, Current>(0);
+        ScalarValue w  = variable_list.template get_value<Scalar, LHS>(4);
+        ScalarGrad  wx = variable_list.template get_gradient<Scalar, LHS>(4);
+        const ScalarValue e = dealii::compare_and_apply_mask<dealii::SIMDComparison::greater_than>(
+          c, ScalarValue(60.0), ScalarValue(2.0), ScalarValue(1.0));
+        variable_list.set_value_term(4, w);
+        variable_list.set_gradient_term(4, D * e * wx);
       }
   }
 

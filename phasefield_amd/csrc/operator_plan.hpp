@@ -109,14 +109,14 @@ namespace ppf
     Undecided ///< compare again at the next application
   };
 
-  /// Zero against zero says nothing of a coupled plan's coefficients (a solve from zero begins
-  /// with such an application).  Plans of the split path have always been taken then: fields at
-  /// rest would be compared in every increment.
+  /// Zero against zero says nothing of the coefficients: applications to zero, of a lhs or a
+  /// coupled plan, are compared again.  (A right-hand side of the split path is taken then:
+  /// fields at rest would be compared in every increment.)
   inline PlanCheck
-  check_plan(const SplitPlan &plan, double worst, double scale, double tol)
+  check_plan(const SplitPlan &plan, bool lhs, double worst, double scale, double tol)
   {
     if (scale == 0.0 && worst == 0.0)
-      return plan.coupled ? PlanCheck::Undecided : PlanCheck::Agrees;
+      return plan.coupled || lhs ? PlanCheck::Undecided : PlanCheck::Agrees;
     return worst <= tol * scale ? PlanCheck::Agrees : PlanCheck::Differs;
   }
 

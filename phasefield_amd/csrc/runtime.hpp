@@ -977,7 +977,7 @@ namespace ppf
               if (!halted_now)
                 {
                   const double    tol   = std::is_same_v<number, float> ? 1e-4 : 1e-11;
-                  const PlanCheck check = check_plan(plan, worst, scale, tol);
+                  const PlanCheck check = check_plan(plan, lhs, worst, scale, tol);
                   entry.verified        = check != PlanCheck::Undecided;
                   if (check == PlanCheck::Differs)
                     {
@@ -2334,6 +2334,24 @@ namespace ppf
                              false);
     }
 
+    /// First use of the plan of a block's lhs in a solve: compared on the block's right-hand
+    /// side, before a preconditioner, a diagonal or a captured V-cycle is made from it.  (The
+    /// solve itself begins with applications to zero, inhomogeneous values and start, that
+    /// every plan agrees on.)
+    void
+    check_lhs_plan(int b)
+    {
+      if (path != OperatorPath::Auto)
+        return;
+      const PlanEntry &entry = split_plan<double>(b, true);
+      if (!entry.verified && (entry.plan.eligible ||
+                              (generic_cell_block && takes_coupled(entry.plan, fine))))
+        {
+          LinearState &ls = linear_state(b);
+          vmult_fine(b, ls.tmp.get(), ls.rhs.get());
+        }
+    }
+
     /// LinearSolver::solve_impl (reference linear_solver.h:305-345).
     SolveStats
     solve_linear(int b)
@@ -2345,6 +2363,7 @@ namespace ppf
       // rhs = scaling * rhs operator
       apply_operator<double>(b, false, fine_fields(), {}, split_block(ls.rhs.get(), b, fine), sc,
                              dirichlet_zero, false);
+      check_lhs_plan(b);
       // inhomogeneous values: g at Dirichlet nodes, 0 elsewhere
       {
         int k = 0;
@@ -2429,6 +2448,7 @@ namespace ppf
           unconverged = ns.residual > ns.tolerance;
           if (!unconverged)
             continue;
+          check_lhs_plan(b);
           // J du = r, from the previous update (level operators see the current
           // solution through the injected fields and re-evaluated diagonals).
           prepare_preconditioner(b);

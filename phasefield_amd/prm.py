@@ -262,7 +262,7 @@ def mechanics(size=100.0, refinement=6, E=2.0, nu=0.3, tolerance=1e-10,
 
 
 def switching(size=8.0, refinement=4, steps=6, dt=2e-3, D=1.0, c_low=-10.0, c_high=70.0,
-              outputs=1):
+              outputs=1, preconditioner="None"):
     """Routing test bed (apps/switching): the initial c ramps from c_low to c_high along
     x, so the value branches of its flux coefficients (c > 1, c > 60) are taken in part of
     the domain."""
@@ -272,6 +272,13 @@ def switching(size=8.0, refinement=4, steps=6, dt=2e-3, D=1.0, c_low=-10.0, c_hi
         f"set Model constant D = {D!r}, DOUBLE",
         f"set Model constant c_low = {c_low!r}, DOUBLE",
         f"set Model constant c_high = {c_high!r}, DOUBLE",
+        "subsection linear solver parameters: 0",
+        "  set solver_ids = 4",
+        "  set tolerance type = AbsoluteResidual",
+        "  set tolerance value = 1e-10",
+        "  set max iterations = 1000",
+        f"  set preconditioner = {preconditioner}",
+        "end",
     ]) + "\n"
 
 

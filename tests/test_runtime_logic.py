@@ -68,10 +68,10 @@ def test_transfers_read_only_what_their_outputs_take(logic, degree):
     assert logic[f"taps_q{degree}"] == "0 0 0 0"
 
 
-def test_comparison_of_zero_with_zero_checks_no_coupled_plan(logic):
+def test_comparison_of_zero_with_zero_decides_nothing(logic):
     # 0 agrees, 1 differs, 2 undecided
-    assert logic["check_split"] == "010111"
-    assert logic["check_coupled"] == "012111"
+    assert logic["check_rhs"] == "010111"
+    assert logic["check_lhs"] == logic["check_coupled"] == "012111"
 
 
 def test_comparison_is_kept_by_the_same_path_only(logic):
