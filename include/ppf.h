@@ -107,7 +107,7 @@ int ppf_field_name(ppf_ctx *ctx, int field, char *buf, int len);
  * with two stencil operands node by node (auto: 1000000, in 2-D 500000, and 100000; both
  * 100000 while one of the four options before is set; 0: tiles at any size);
  * "stencil_store_policy" = auto|temporal|nontemporal sets the cache policy of
- * its output stores (auto: non-temporal when the launch's arrays exceed 256 MiB);
+ * its output stores (auto: non-temporal when the arrays the launch reads exceed 150 MiB);
  * "generic_kernel" = cell_block|two_pass selects the generic path's kernels (cell_block:
  * one launch, cell blocks staged in shared memory, no device scratch; two_pass: a cell
  * kernel into a device scratch array and a node gather; cell_block falls back to

@@ -1093,10 +1093,7 @@ namespace ppf
             }
           a.keep_dirichlet = out.dirichlet_write == dirichlet_value ? 1 : 0;
           a.halt           = out.halt;
-          const int64_t footprint = 6 * g.n_nodes * int64_t(sizeof(number));
-          a.nt_store = stencil_store_policy == StorePolicy::NonTemporal ||
-                       (stencil_store_policy == StorePolicy::Auto &&
-                        footprint > stencil_nt_min_bytes);
+          a.nt_store = stores_nontemporally(3 * g.n_nodes * int64_t(sizeof(number)));
           // Tile shape: the fewest workgroups, halo staging counted at a quarter of a
           // thread's work; a lattice of 129 nodes takes 43 columns x 10 rows, where tiles
           // of 64 columns would leave a third of the lanes idle.  At least 32 columns, so
@@ -1423,9 +1420,7 @@ namespace ppf
       // 32-bit byte offsets in the kernel: arrays up to 4 GiB.
       if (int64_t(a.n[0]) * a.n[1] * a.n[2] * int64_t(sizeof(ST)) > (int64_t(1) << 32))
         return false;
-      // Store policy: non-temporal when the distinct arrays the launch reads and writes exceed
-      // the 256 MB Infinity Cache (stencil_nt_min_bytes): beyond it the output would not be
-      // there for the launch that reads it.
+      // Store policy by the distinct arrays that the launch reads (stores_nontemporally).
       {
         const void *arrays[stencil_max_ops + PPF_MAX_FIELDS * (PPF_N_SLOTS + 1)];
         int         n_arrays = 0;
@@ -1438,17 +1433,10 @@ namespace ppf
         for (int k = 0; k < a.n_ops; ++k)
           add(a.op[k]);
         for (int f = 0; f < PPF_MAX_FIELDS; ++f)
-          {
-            for (int s = 0; s < PPF_N_SLOTS; ++s)
-              if (deps.flags[f][s] & slot_values)
-                add(a.val[f][s]);
-            if (out.out_mask & (1u << f))
-              add(out.dst[f]);
-          }
-        const int64_t footprint = int64_t(n_arrays) * g.n_nodes * int64_t(sizeof(ST));
-        a.nt_store = stencil_store_policy == StorePolicy::NonTemporal ||
-                     (stencil_store_policy == StorePolicy::Auto &&
-                      footprint > stencil_nt_min_bytes);
+          for (int s = 0; s < PPF_N_SLOTS; ++s)
+            if (deps.flags[f][s] & slot_values)
+              add(a.val[f][s]);
+        a.nt_store = stores_nontemporally(int64_t(n_arrays) * g.n_nodes * int64_t(sizeof(ST)));
       }
       // A pending coarse-grid solve takes this operator (src = p, dst = ap) and runs the
       // whole CG in one workgroup instead of one launch per vector operation.
@@ -2105,12 +2093,7 @@ namespace ppf
           if (nblocks >= (int64_t(1) << 31) || nrem >= (int64_t(1) << 31))
             return pair_skip(ba, __LINE__);
           a.n_blocks = int(nblocks);
-          {
-            const int64_t footprint = 4 * fine.n_nodes * int64_t(sizeof(double));
-            a.nt_store = stencil_store_policy == StorePolicy::NonTemporal ||
-                         (stencil_store_policy == StorePolicy::Auto &&
-                          footprint > stencil_nt_min_bytes);
-          }
+          a.nt_store = stores_nontemporally(2 * fine.n_nodes * int64_t(sizeof(double)));
           if (probe_req.pending && probe_req.block == bb && a.n_blocks > 0)
             {
               a.probe_result = probe_req.result;
@@ -4263,17 +4246,26 @@ namespace ppf
     int64_t                                n_cus_     = 0;
     int64_t                                lds_limit_ = 0;
     int                                    stencil_target_blocks = 2048;
-    /// Cache policy of the stencil kernel's output stores (Auto: non-temporal for launches
-    /// whose arrays exceed stencil_nt_min_bytes, the size of the Infinity Cache).  Measured,
-    /// temporal / non-temporal, launches that read each other's output, by the bytes of a
-    /// launch: four Poisson Q2 applications (FP64) 214 MiB 53.9 / 61.5 us each, 259 MiB 71.5 /
-    /// 73.0, 284 MiB 91.1 / 90.6, 368 MiB 112 / 109; the coupled stencil 254 MiB 94.3 / 99.2, 329
-    /// MiB 121.5 / 121.9.  Increments, by the line drawn at 192 / 256 / 384 MiB: Cahn-Hilliard
-    /// 104^3 cells 105.7 / 90.4 / 90.1 us, 128^3 141.1 / 136.4 / 154.6; precipitate 224^3 168.6 /
-    /// 168.4 / 192.5, 256^3 218 / 218 / 247.5, 192^3 the same.  An output that nothing reads next is
-    /// better stored non-temporally above 230 MiB: 259 MiB 65.4 / 62.1, 310 MiB 91.6 / 66.5.
-    StorePolicy                            stencil_store_policy = StorePolicy::Auto;
-    int64_t                                stencil_nt_min_bytes = int64_t(256) << 20;
+    /// Cache policy of the stencil kernels' output stores.  Auto: non-temporal where the arrays
+    /// that the launch reads exceed stencil_nt_read_bytes.  What it reads passes through the 256
+    /// MB Infinity Cache too, and above that too little of the output is left there for the
+    /// launch that reads it.  Measured, temporal / non-temporal, launches that read each other's
+    /// output, by the MiB that one reads: four Poisson Q2 applications FP64 107 53.9 / 61.5 us
+    /// each, 130 (257^3 nodes) 71.5 / 73.0, 142 91.1 / 90.6, 155 93.7 / 92.4, 184 112 / 109; FP32
+    /// 126 79.4 / 90.1, 146 98.6 / 103.1, 168 105.3 / 108.5; the coupled stencil 127 94.3 / 99.2, 165
+    /// 121.5 / 121.9.  Cahn-Hilliard increments (the c block reads two arrays, the mu block one):
+    /// 96^3 cells (108) 66.7 / 71.7, 104^3 (138) 90.1 / 105.4, 112^3 (172) 117.2 / 115.2, 144^3 (mu 182)
+    /// 232.7 / 224.5; precipitate: 192^3 (108) 109.8 / 111.4, 208^3 (137) 156 / 154, 224^3 (172) 192.5 /
+    /// 168.5, 256^3 (256) 247.5 / 217.9.  An output that nothing reads next is better stored
+    /// non-temporally from about 115 MiB on: 130 65.4 / 62.1, 155 91.6 / 66.5.
+    StorePolicy                            stencil_store_policy  = StorePolicy::Auto;
+    int64_t                                stencil_nt_read_bytes = int64_t(150) << 20;
+    bool
+    stores_nontemporally(int64_t bytes_read) const
+    {
+      return stencil_store_policy == StorePolicy::NonTemporal ||
+             (stencil_store_policy == StorePolicy::Auto && bytes_read > stencil_nt_read_bytes);
+    }
     /// Lattices with fewer nodes run split operators column by column, with two stencil
     /// operands node by node, instead of by marching tiles (launch_stencil): option
     /// stencil_min_nodes sets both limits (-1: by size, column_limit and node_limit).
