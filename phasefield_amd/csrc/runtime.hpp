@@ -4233,9 +4233,10 @@ namespace ppf
     int                                    stencil_waves   = 0;
     int                                    stencil_z_chunk = 0;
     /// Workgroup -> tile order of the stencil kernel (StencilArgs::map_mode; -1: by size).
-    /// On large lattices a band of tile rows per XCD keeps the rows and planes that tiles
-    /// share in its L2: precipitate Q1 at 7.1M nodes 126.2 -> 120.6 us per increment, Poisson
-    /// Q2 at 17M 83.6 -> 79.5 us per application; at 2.1M nodes (Cahn-Hilliard) 31.6 -> 31.9.
+    /// On large lattices a band of tile rows per XCD is faster: precipitate Q1 at 7.1M nodes
+    /// 126.2 -> 120.6 us per increment, Poisson Q2 at 17M 73.7 -> 71.1 us per chained application;
+    /// at 2.1M nodes (Cahn-Hilliard) 31.6 -> 31.9.  Not by L2 reuse: at 17M nodes the launch
+    /// fetches 239 MB past the L2s in bands, 215 in linear order.
     int                                    stencil_map     = -1;
     static constexpr int64_t               stencil_band_nodes = int64_t(4) << 20;
     /// Generic path kernel: the one-pass cell-block kernel (true) or the two-pass
