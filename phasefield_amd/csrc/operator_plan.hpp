@@ -23,6 +23,7 @@
 #include <prismspf/core/dependencies.h>
 #include <prismspf/core/solve_block.h>
 
+#include <algorithm>
 #include <cmath>
 #include <random>
 #include <sstream>
@@ -106,18 +107,25 @@ namespace ppf
   {
     Agrees,
     Differs,
-    Undecided ///< compare again at the next application
+    Undecided ///< zero against zero, which says nothing of the coefficients
   };
 
-  /// Zero against zero says nothing of the coefficients: applications to zero, of a lhs or a
-  /// coupled plan, are compared again.  (A right-hand side of the split path is taken then:
-  /// fields at rest would be compared in every increment.)
   inline PlanCheck
-  check_plan(const SplitPlan &plan, bool lhs, double worst, double scale, double tol)
+  check_plan(double worst, double scale, double tol)
   {
     if (scale == 0.0 && worst == 0.0)
-      return plan.coupled || lhs ? PlanCheck::Undecided : PlanCheck::Agrees;
+      return PlanCheck::Undecided;
     return worst <= tol * scale ? PlanCheck::Agrees : PlanCheck::Differs;
+  }
+
+  /// Applications of a coupled operator that the generic path takes, without a comparison,
+  /// after the n-th comparison of zero with zero: none after the first (the next application
+  /// of a solve is to something), then twice as many each time, so that a program that keeps
+  /// applying the operator to zero does not wait for a comparison each time.
+  inline unsigned int
+  applications_until_check(unsigned int n)
+  {
+    return (1u << std::min(n, 20u)) - 2u;
   }
 
   /// Whether a plan derived anew (another time step, time or increment) keeps the comparison of

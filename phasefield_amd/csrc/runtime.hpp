@@ -674,6 +674,12 @@ namespace ppf
       unsigned int increment = 0;
       /// The split path was compared with the generic path on real fields (first use).
       bool verified = false;
+      /// The comparison was of zero with zero: good enough for applications of a split
+      /// operator (fields at rest would be compared in every increment), not for a solve.
+      bool by_zero = false;
+      /// Coupled plans: comparisons of zero with zero so far, and applications left to the
+      /// generic path before the next comparison.
+      unsigned int zeros = 0, skip = 0;
     };
 
     /// The split plan of block b's rhs or lhs, re-derived when the time step changes and,
@@ -709,7 +715,12 @@ namespace ppf
           entry.verified      = true;
         }
       else if (it != plans.end())
-        entry.verified = it->second.verified && keeps_check(it->second.plan, entry.plan);
+        {
+          entry.verified = it->second.verified && keeps_check(it->second.plan, entry.plan);
+          entry.by_zero  = it->second.by_zero;
+          entry.zeros    = it->second.zeros;
+          entry.skip     = it->second.skip;
+        }
       return plans[key] = entry, plans[key];
     }
 
@@ -910,7 +921,7 @@ namespace ppf
         for (const number *sp : src)
           in_place = in_place || sp == d;
       if ((use_split || use_coupled) && path == OperatorPath::Auto && !entry.verified &&
-          lf.grid == &fine && !in_place && !(use_coupled && capturing()))
+          lf.grid == &fine && !in_place && !(use_coupled && (entry.skip > 0 || capturing())))
         {
           const int64_t n   = g.n_nodes;
           number       *ref = nullptr;
@@ -977,8 +988,11 @@ namespace ppf
               if (!halted_now)
                 {
                   const double    tol   = std::is_same_v<number, float> ? 1e-4 : 1e-11;
-                  const PlanCheck check = check_plan(plan, lhs, worst, scale, tol);
-                  entry.verified        = check != PlanCheck::Undecided;
+                  const PlanCheck check = check_plan(worst, scale, tol);
+                  entry.by_zero         = check == PlanCheck::Undecided;
+                  entry.verified        = !(entry.by_zero && use_coupled);
+                  if (entry.by_zero && use_coupled)
+                    entry.skip = applications_until_check(++entry.zeros);
                   if (check == PlanCheck::Differs)
                     {
                       std::ostringstream msg;
@@ -1002,9 +1016,11 @@ namespace ppf
             }
         }
       // A coupled plan that could not be compared (an operand in place, a stream under
-      // capture, too little borrowed scratch) leaves the application to the generic path that
-      // such operators always had.  (Levels have no comparison: their operators only
-      // precondition.)
+      // capture, too little borrowed scratch, zero operands before) leaves the application to
+      // the generic path that such operators always had.  (Levels have no comparison: their
+      // operators only precondition.)
+      if (lf.grid == &fine && entry.skip > 0)
+        --entry.skip;
       launch(use_split || (use_coupled && (entry.verified || lf.grid != &fine)), out);
     }
 
@@ -2326,11 +2342,13 @@ namespace ppf
     {
       if (path != OperatorPath::Auto)
         return;
-      const PlanEntry &entry = split_plan<double>(b, true);
-      if (!entry.verified && (entry.plan.eligible ||
-                              (generic_cell_block && takes_coupled(entry.plan, fine))))
+      PlanEntry &entry = split_plan<double>(b, true);
+      if ((!entry.verified || entry.by_zero) &&
+          (entry.plan.eligible || (generic_cell_block && takes_coupled(entry.plan, fine))))
         {
           LinearState &ls = linear_state(b);
+          entry.verified  = false;
+          entry.skip      = 0;
           vmult_fine(b, ls.tmp.get(), ls.rhs.get());
         }
     }

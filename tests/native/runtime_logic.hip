@@ -102,18 +102,15 @@ main()
             << refused(lattice(46341, 46340, 1), lattice(92681, 92679, 1)) << "\n"
             << "transfer_planes: " << refused(lattice(2, 2, 40000), lattice(3, 3, 79999)) << "\n";
   // comparisons: in agreement, apart, zero with zero, nothing with something, not finite
-  for (int kind = 0; kind < 3; ++kind)
-    {
-      ppf::SplitPlan plan;
-      plan.eligible = kind < 2;
-      plan.coupled  = kind == 2;
-      std::cout << (kind == 0 ? "check_rhs: " : kind == 1 ? "check_lhs: " : "check_coupled: ");
-      const double inf = std::numeric_limits<double>::infinity();
-      for (auto [worst, scale] : {std::pair {1e-13, 2.0}, {1e-3, 2.0}, {0.0, 0.0}, {1e-30, 0.0},
-                                  {inf, 2.0}, {inf, 0.0}})
-        std::cout << int(ppf::check_plan(plan, kind == 1, worst, scale, 1e-11));
-      std::cout << "\n";
-    }
+  std::cout << "check: ";
+  const double inf = std::numeric_limits<double>::infinity();
+  for (auto [worst, scale] : {std::pair {1e-13, 2.0}, {1e-3, 2.0}, {0.0, 0.0}, {1e-30, 0.0},
+                              {inf, 2.0}, {inf, 0.0}})
+    std::cout << int(ppf::check_plan(worst, scale, 1e-11));
+  std::cout << "\ncheck_again: ";
+  for (unsigned int n : {1u, 2u, 3u, 4u, 20u, 4000000000u})
+    std::cout << ppf::applications_until_check(n) << " ";
+  std::cout << "\n";
   // plans derived anew: split, coupled and generic before, each followed by each
   std::cout << "keeps_check: ";
   for (int before = 0; before < 3; ++before)

@@ -168,19 +168,27 @@ def test_small_scratch_compares(device):
     assert rel_err(dst.cpu().numpy(), ref.cpu().numpy()) <= 1e-13
 
 
-def test_zero_operand_checks_nothing(device):
+@pytest.mark.parametrize("zeros, until", [(1, 1), (2, 3), (5, 7), (9, 3)])
+def test_zero_operand_checks_nothing(device, zeros, until):
     """An application to zero agrees whatever the coefficients are: the inverse diagonal is
-    probed on the generic path (its bits) until an application to something has agreed."""
+    probed on the generic path (its bits) until an application to something has been compared,
+    the next one after one application to zero, at the latest the `until`-th after more."""
     import torch
 
     fast, slow, src = fresh_pair((6, 5, 4), device, torch)
     diag, ref = torch.empty_like(src), torch.empty_like(src)
     slow.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, ref.data_ptr())
-    for _ in range(2):
+    generic = apply(slow, torch, src, OP_LHS, SCALE_NONE, FP64)
+    for _ in range(zeros):
         assert not apply(fast, torch, torch.zeros_like(src), OP_LHS, SCALE_NONE, FP64).any()
         fast.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, diag.data_ptr())
         assert torch.equal(diag, ref)
-    apply(fast, torch, src, OP_LHS, SCALE_NONE, FP64)
+    for k in range(until):
+        fast.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, diag.data_ptr())
+        assert torch.equal(diag, ref)
+        got = apply(fast, torch, src, OP_LHS, SCALE_NONE, FP64)
+        assert np.array_equal(got, generic) == (k < until - 1)
+        assert rel_err(got, generic) <= 1e-13
     fast.inverse_diagonal(1, SCALE_INVM_SQRT, FP64, diag.data_ptr())
     assert not torch.equal(diag, ref)  # from the coefficients
     assert float(((diag - ref).abs() / ref.abs()).max()) <= 1e-13

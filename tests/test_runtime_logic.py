@@ -70,8 +70,9 @@ def test_transfers_read_only_what_their_outputs_take(logic, degree):
 
 def test_comparison_of_zero_with_zero_decides_nothing(logic):
     # 0 agrees, 1 differs, 2 undecided
-    assert logic["check_rhs"] == "010111"
-    assert logic["check_lhs"] == logic["check_coupled"] == "012111"
+    assert logic["check"] == "012111"
+    # the next application compares again, then fewer and fewer
+    assert logic["check_again"].split() == ["0", "2", "6", "14", "1048574", "1048574"]
 
 
 def test_comparison_is_kept_by_the_same_path_only(logic):
