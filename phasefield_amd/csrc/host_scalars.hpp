@@ -25,14 +25,22 @@ namespace ppf
       : tag(last_tag)
     {}
 
-    /// Tag of the next scalar (1 .. 2^31 - 1).  Its entry is emptied: pinned memory comes with
-    /// any contents, such as the entries of an earlier context, whose tags began at 1 too and
-    /// would be taken for the scalars of this one.
+    /// Empties the entries before the first use: pinned memory comes with any contents, such
+    /// as the entries of an earlier context, whose tags began at 1 too and would be taken for the
+    /// scalars of this one.  (Later an entry holds a tag of this ring, an older one than is
+    /// awaited there.)
+    static void
+    clear(HostScalar *entries)
+    {
+      for (int k = 0; k < size; ++k)
+        *reinterpret_cast<volatile unsigned int *>(&entries[k].word) = 0u;
+    }
+
+    /// Tag of the next scalar, 1 .. 2^31 - 1.
     unsigned int
-    issue(HostScalar *entries)
+    issue()
     {
       tag = tag % 0x7fffffffu + 1u;
-      *reinterpret_cast<volatile unsigned int *>(&entry(entries, tag)->word) = 0u;
       return tag;
     }
 

@@ -205,7 +205,7 @@ namespace ppf
       fine = make_grid(inputs.spatial_discretization.global_refinement);
       PPF_HIP_CHECK(hipStreamCreate(&stream));
       reduce_buf.resize(2 * reduce_blocks + 8);
-      (void) host_scalars.get(HostScalarRing::size); // not in the first solve or comparison
+      HostScalarRing::clear(host_scalars.get(HostScalarRing::size));
       coarse_slots.resize(8);
       coarse_flag.resize(1);
       halt_flag.resize(max_pipeline_depth + 1);
@@ -615,7 +615,7 @@ namespace ppf
     unsigned int
     next_host_tag()
     {
-      return host_ring.issue(host_scalars.get(HostScalarRing::size));
+      return host_ring.issue();
     }
 
     HostScalar *

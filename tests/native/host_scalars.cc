@@ -14,11 +14,12 @@ main()
     *HostScalarRing::entry(entries, t) = {100.0 + t, t << 1};
 
   HostScalarRing ring;
+  HostScalarRing::clear(entries);
   int            stale = 0, missed = 0;
   unsigned int   first = 0;
   for (int k = 0; k < 9; ++k)
     {
-      const unsigned int t = ring.issue(entries);
+      const unsigned int t = ring.issue();
       if (k == 0)
         first = t;
       HostScalar *e = HostScalarRing::entry(entries, t);
@@ -30,7 +31,7 @@ main()
 
   // an emptied entry is no tag's, also where the tags start again
   HostScalarRing late(0x7ffffffeu);
-  const unsigned a = late.issue(entries), b = late.issue(entries);
+  const unsigned a = late.issue(), b = late.issue();
   std::cout << "last: " << a << "\nwrapped: " << b << "\nempty: "
             << HostScalarRing::ready(HostScalarRing::word(HostScalarRing::entry(entries, b)), b)
             << "\n";
